@@ -7,6 +7,8 @@
 #include <hip/hip_fp16.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "../../include/miattn.h"
 
 namespace miattn {
@@ -72,6 +74,27 @@ __device__ __forceinline__ void store16(void* p, const uint4& v) {
   *reinterpret_cast<uint4*>(p) = v;
 }
 
+// 16 / sizeof(T) fp32 values -> one 16-byte vector of T (round-to-nearest-even for 16-bit types).
+template <typename T>
+__device__ __forceinline__ uint4 pack16(const float* v) {
+  if constexpr (sizeof(T) == 4) {
+    return make_uint4(__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]),
+                      __float_as_uint(v[3]));
+  } else {
+    uint32_t w[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if constexpr (std::is_same<T, bf16_t>::value) {
+        typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+        w[i] = __builtin_bit_cast(uint32_t, bf16x2{(__bf16)v[2 * i], (__bf16)v[2 * i + 1]});
+        continue;
+      }
+      w[i] = uint32_t(from_f32<T>(v[2 * i]).bits) | (uint32_t(from_f32<T>(v[2 * i + 1]).bits) << 16);
+    }
+    return make_uint4(w[0], w[1], w[2], w[3]);
+  }
+}
+
 // Sum over s = 0 .. parts-1 (parts >= 1) of f[s * plane], added in that order in fp32 (the
 // split-K partial sums of one output element), split into a load and a sum step so a kernel
 // can issue the loads of all its elements before any arithmetic (an empty asm in a rounding
@@ -135,6 +158,10 @@ constexpr int kDppRowRor8 = 0x128;
 __device__ __forceinline__ float swap16(float x) {
   return __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(x), 0x401F));
 }
+// Exchange with lane ^ 4, likewise.
+__device__ __forceinline__ float swap4(float x) {
+  return __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(x), 0x101F));
+}
 // Exchange with lane ^ 32: gfx950 v_permlane32_swap.
 __device__ __forceinline__ float swap32(float x) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
@@ -181,6 +208,50 @@ template <typename T>
 __device__ __forceinline__ float rt(float x) {
   asm volatile("" : "+v"(x));
   return to_f32(from_f32<T>(x));
+}
+
+// rt of eight values at once, in place; returns them packed (one packed conversion and two
+// unpacking ops per pair). bf16 has no native arithmetic that a rounding could fold into, so
+// it needs no asm in between.
+template <typename T>
+__device__ __forceinline__ uint4 rt8(float (&v)[8]) {
+  if constexpr (std::is_same<T, f16_t>::value) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) asm("" : "+v"(v[j]));
+  }
+  const uint4 w = pack16<T>(v);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) v[j] = Vec16<T>::get(w, j);
+  return w;
+}
+
+// rt<T>(x[j] / d) for eight x and one d, all of them T values, without a division each; returned in x.
+// x / d is never close enough to a rounding boundary of T for the shorter form to round the
+// other way: with p-bit significands (8 for bf16, 11 for fp16) a boundary m has p + 1 bits, so
+// |x / d - m| = |x - m d| / d is at least 2^-(2p + 1) relative (it is not 0: m d has more than
+// p significant bits). x * (1/d) is within 2^-23, enough for bf16's 2^-17; fp16's 2^-23 takes
+// one correction by the exact remainder (within 2^-46 before its rounding). A d whose
+// reciprocal could overflow takes the divisions (wave-uniform, not seen with a usual eps).
+template <typename T>
+__device__ __forceinline__ void div_rt8(float (&x)[8], float d) {
+  if (__any(!(d > 0x1p-100f))) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = x[j] / d;
+  } else {
+    const float r = 1.0f / d;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      float q = x[j] * r;
+      // 0x198: a finite non-zero quotient (the others are final, and the correction would lose the
+      // sign of a zero and turn an infinity into NaN)
+      if constexpr (std::is_same<T, f16_t>::value) {
+        const float fixed = fmaf(fmaf(-q, d, x[j]), r, q);
+        q = __builtin_amdgcn_classf(q, 0x198) ? fixed : q;
+      }
+      x[j] = q;
+    }
+  }
+  rt8<T>(x);
 }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }

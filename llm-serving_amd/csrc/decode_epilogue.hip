@@ -33,6 +33,7 @@
 // of 64 and in lane l ^ 32 when it is 32. The projection rows are T, or fp32 split-K partial
 // sums [parts][B][row_stride] of mi_rows_gemm, summed in split order and rounded once to T
 // (the value the projection's own output would hold).
+#include <initializer_list>
 #include <type_traits>
 
 #include "common.h"
@@ -182,6 +183,137 @@ __global__ __launch_bounds__(256) void qk_norm_rope_write_kernel(
   }
 }
 
+// The same epilogue over a T projection (no partial sums) with 16-byte accesses, for 16-bit
+// types: a head is D / 8 consecutive lanes, lane c holding elements 8c .. 8c + 7, and a
+// workgroup walks one row's heads, so position, slot, RoPE entries and norm weights are
+// loaded once per row instead of once per (row, head). Bound by memory: a packed group of T
+// tokens moves T x (2 H + 6 H_kv) x D values. Measured (bf16, graph replay, with the packed k/v
+// copies) against the kernel above, which moves one 2-byte element per lane per access and
+// divides for each: 8192 tokens at H 16 / H_kv 8 / D 128 82.7 -> 37.2 us (168 MB, 4.5 TB/s; a
+// large copy reaches 5.1), at 8 / 2 / 256 47.7 -> 33.3, 4311 tokens 44.0 -> 22.8. The
+// projection is read and the pool written with the nontemporal hint (39.2 -> 37.2 us at 8192
+// tokens): the next reader of either is far away; q_out, k_out and v_out are the attention's
+// next input and stay cached.
+//
+// Bit-equal to the kernel above: its lane l sums the squares of elements l, l + 64, ... in that
+// order and then runs the 64-lane butterfly l ^ 1, ^ 2, ... ^ 32. Here the elements l + 64 j of
+// one l are in lanes c, c + 8, .. (c = l / 8), added in the same order by head_squares(); the
+// butterfly's first three levels are the in-lane tree over the 8 elements and the last three
+// an 8-lane butterfly over c.
+template <int D>
+__device__ __forceinline__ float head_squares(const float (&sq)[8], int c) {
+  float v[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    if constexpr (D == 64) {
+      v[j] = sq[j];
+    } else if constexpr (D == 128) {
+      v[j] = sq[j] + dpp<kDppRowRor8>(sq[j]);
+    } else {
+      // ((a0 + a1) + a2) + a3 of lanes c, c + 8, c + 16, c + 24 (c < 8), in every one of them
+      const float far = swap16(sq[j]);
+      const float low = (c & 16) ? far : sq[j], high = (c & 16) ? sq[j] : far;
+      const float high8 = dpp<kDppRowRor8>(high);
+      v[j] = ((low + dpp<kDppRowRor8>(low)) + ((c & 8) ? high8 : high)) + ((c & 8) ? high : high8);
+    }
+  }
+  return group_allreduce<8, SumOp>(((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7])));
+}
+
+template <typename T, int D, typename IdxT>
+__global__ __launch_bounds__(256) void qk_norm_rope_write_vec_kernel(
+    const T* __restrict__ qkv, int64_t row_stride, const T* __restrict__ q_w, const T* __restrict__ k_w,
+    const T* __restrict__ cos_tab, const T* __restrict__ sin_tab, int64_t n_pos, int rotary,
+    const int64_t* __restrict__ pos, const IdxT* __restrict__ slots, T* __restrict__ q_out, T* __restrict__ k_pool,
+    T* __restrict__ v_pool, T* __restrict__ k_out, T* __restrict__ v_out, int H, int H_kv, int64_t n_slots, float eps,
+    int norm_mode, int32_t* __restrict__ err) {
+  constexpr int E = 8, LPH = D / E, HPW = 256 / LPH;  // lanes per head, heads per workgroup pass
+  const int c = threadIdx.x % LPH;
+  const int b = blockIdx.x;
+  const int n_heads = H + 2 * H_kv;
+  const int step = HPW * gridDim.y;
+  const int head0 = blockIdx.y * HPW + threadIdx.x / LPH;
+  const int64_t pb = pos[b];
+  const IdxT slot = slots[b];
+  const T* src = qkv + int64_t(b) * row_stride + c * E;
+  // the row of each output a head goes to; k and v of a row that is written go to the pool and,
+  // when asked for, to the packed copy
+  auto packed_row = [&](int head) -> T* {
+    if (head < H) return q_out + (int64_t(b) * H + head) * D + c * E;
+    T* out = head < H + H_kv ? k_out : v_out;
+    return out == nullptr ? nullptr : out + (int64_t(b) * H_kv + (head - H) % H_kv) * D + c * E;
+  };
+  const bool idle = slot == IdxT(-1);
+  if (idle || pb < 0 || pb >= n_pos || !(slot >= 0 && int64_t(slot) < n_slots)) {  // uniform: see the kernel above
+    if (!idle && blockIdx.y == 0 && threadIdx.x == 0 && err != nullptr) atomicCAS(err, 0, b + 1);
+    for (int head = head0; head < n_heads; head += step) {
+      T* row = packed_row(head);
+      if (row != nullptr) store16(row, make_uint4(0u, 0u, 0u, 0u));
+    }
+    return;
+  }
+  const int half = rotary >> 1;  // 32, 64 or 128: a lane's 8 elements are on one side of it
+  const int e0 = c * E;
+  const int a0 = e0 < half ? e0 : (e0 < rotary ? e0 - half : 0);
+  const uint4 cv = load16(cos_tab + pb * half + a0), sv = load16(sin_tab + pb * half + a0);
+  const uint4 wq = load16(q_w + e0), wk = load16(k_w + e0);
+
+  auto finish = [&](int head, const uint4& raw) {
+    uint4 result = raw;  // a v head is copied as it is
+    if (head < H + H_kv) {
+      const uint4 w = head < H ? wq : wk;
+      float x[E], sq[E];
+#pragma unroll
+      for (int j = 0; j < E; ++j) {
+        x[j] = Vec16<T>::get(raw, j);
+        sq[j] = x[j] * x[j];  // exact: a product of 16-bit values
+      }
+      if (norm_mode == kNormQwen3) {
+        rt8<T>(sq);
+        const float ms = rt<T>(head_squares<D>(sq, c) * (1.0f / D));
+        div_rt8<T>(x, rt<T>(sqrtf(rt<T>(ms + eps))));
+#pragma unroll
+        for (int j = 0; j < E; ++j) x[j] *= Vec16<T>::get(w, j);
+      } else {
+        const float r = 1.0f / sqrtf(head_squares<D>(sq, c) * (1.0f / D) + eps);
+#pragma unroll
+        for (int j = 0; j < E; ++j) x[j] = (x[j] * r) * (1.0f + Vec16<T>::get(w, j));
+      }
+      result = rt8<T>(x);  // the normed head
+      if (e0 < rotary || half == 128) {
+        // the rotation partner is this element of lane c ^ (half / 8); the first half's lanes take
+        // x cos - partner sin, the second's partner sin + x cos
+        float p[E];
+#pragma unroll
+        for (int j = 0; j < E; ++j) {
+          p[j] = half == 64 ? dpp<kDppRowRor8>(x[j]) : half == 32 ? swap4(x[j]) : swap16(x[j]);
+          p[j] *= Vec16<T>::get(sv, j);
+          x[j] *= Vec16<T>::get(cv, j);
+        }
+        rt8<T>(p);
+        rt8<T>(x);
+#pragma unroll
+        for (int j = 0; j < E; ++j) x[j] = e0 < half ? x[j] - p[j] : x[j] + p[j];
+        result = rt8<T>(x);
+      }
+    }
+    T* row = packed_row(head);
+    if (row != nullptr) store16(row, result);
+    if (head >= H) {
+      T* pool = head < H + H_kv ? k_pool : v_pool;
+      store16_nt(pool + (int64_t(slot) * H_kv + (head - H) % H_kv) * D + e0, result);
+    }
+  };
+  // two heads' loads at a time ahead of their arithmetic
+  for (int head = head0; head < n_heads; head += 2 * step) {
+    const int next = head + step;
+    const uint4 r0 = load16_nt(src + int64_t(head) * D);
+    const uint4 r1 = load16_nt(src + int64_t(next < n_heads ? next : head) * D);
+    finish(head, r0);
+    if (next < n_heads) finish(next, r1);
+  }
+}
+
 // Launch arguments shared by every instantiation.
 struct EpilogueArgs {
   const void* qkv; int64_t row_stride; int parts; const void* q_w; const void* k_w; const void* cos_tab;
@@ -190,8 +322,48 @@ struct EpilogueArgs {
   float eps; int norm_mode; int32_t* err; hipStream_t s;
 };
 
+// q/k/v values from which the 16-byte kernel runs: below, a launch is latency, and a lane's
+// eight elements are a longer chain than one or two (H 16 / H_kv 8 / D 128: 32 rows 2.75 against
+// 3.28 us, 128 rows 3.17 against 3.45, 256 rows 4.08 against 4.00, 512 rows 6.3 against 5.4).
+constexpr int64_t kVecValues = 1 << 20;
+// Rows from which one workgroup walks all heads of a row (8192 rows 39.2 against 45.5 us with
+// the heads shared out over the grid's y axis); below, they are shared out so that a small
+// batch still spreads over the chip (300 rows 4.4 against 5.4 us).
+constexpr int kRowPerGroup = 1024;
+
+// Every address the 16-byte kernel touches is a multiple of 16 bytes (rows and heads are
+// multiples of 64 elements; the caller's pointers and row stride are what can be off).
+bool vec16_ok(const EpilogueArgs& a) {
+  uintptr_t all = 0;
+  for (const void* p : {a.qkv, a.q_w, a.k_w, a.cos_tab, a.sin_tab, static_cast<const void*>(a.q_out),
+                        static_cast<const void*>(a.k_pool), static_cast<const void*>(a.v_pool),
+                        static_cast<const void*>(a.k_out), static_cast<const void*>(a.v_out)}) {
+    all |= reinterpret_cast<uintptr_t>(p);
+  }
+  return all % 16 == 0 && a.row_stride % 8 == 0;
+}
+
 template <typename T, int D>
 int launch_d(const EpilogueArgs& a) {
+  if constexpr (sizeof(T) == 2) {
+    if (a.parts == 0 && int64_t(a.B) * (a.H + 2 * a.H_kv) * D >= kVecValues && vec16_ok(a)) {
+      constexpr int HPW = 256 * 8 / D;  // heads per workgroup pass
+      const unsigned groups = (a.H + 2 * a.H_kv + HPW - 1) / HPW;
+      const dim3 grid(a.B, a.B >= kRowPerGroup ? 1 : groups);
+      auto go = [&](auto idx_tag) {
+        using IdxT = decltype(idx_tag);
+        hipLaunchKernelGGL((qk_norm_rope_write_vec_kernel<T, D, IdxT>), grid, dim3(256), 0, a.s,
+                           static_cast<const T*>(a.qkv), a.row_stride, static_cast<const T*>(a.q_w),
+                           static_cast<const T*>(a.k_w), static_cast<const T*>(a.cos_tab),
+                           static_cast<const T*>(a.sin_tab), a.n_pos, a.rotary, a.pos,
+                           static_cast<const IdxT*>(a.slots), static_cast<T*>(a.q_out), static_cast<T*>(a.k_pool),
+                           static_cast<T*>(a.v_pool), static_cast<T*>(a.k_out), static_cast<T*>(a.v_out), a.H, a.H_kv,
+                           a.n_slots, a.eps, a.norm_mode, a.err);
+      };
+      if (a.slot_bits == 32) go(int32_t{}); else go(int64_t{});
+      return launch_status("mi_qk_norm_rope_write");
+    }
+  }
   constexpr int kWaves = 4;
   const dim3 grid(a.B, (a.H + 2 * a.H_kv + kWaves - 1) / kWaves);
   const int64_t plane = int64_t(a.B) * a.row_stride;

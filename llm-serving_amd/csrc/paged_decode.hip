@@ -155,22 +155,6 @@ __device__ __forceinline__ float dot16<float>(const uint4& q, const uint4& k, fl
   return fmaf(__uint_as_float(q.w), __uint_as_float(k.w), acc);
 }
 
-// EPL fp32 values -> one 16-byte vector of T (round-to-nearest-even for 16-bit types).
-template <typename T>
-__device__ __forceinline__ uint4 pack16(const float* v) {
-  if constexpr (sizeof(T) == 4) {
-    return make_uint4(__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]),
-                      __float_as_uint(v[3]));
-  } else {
-    uint32_t w[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      w[i] = uint32_t(from_f32<T>(v[2 * i]).bits) | (uint32_t(from_f32<T>(v[2 * i + 1]).bits) << 16);
-    }
-    return make_uint4(w[0], w[1], w[2], w[3]);
-  }
-}
-
 __device__ __forceinline__ int clamp_len(int len, int capacity) {
   len = len < capacity ? len : capacity;  // page-walk clamp (reference :593)
   return len > 0 ? len : 0;

@@ -1,0 +1,71 @@
+"""The 16-byte kernels that the token ops of a packed group run on (many rows) against the
+kernels that small batches run on: the same op on the same rows, once as one call and once in
+calls of a few rows each, must give the same bits. The small calls are pinned to the
+reference's tensor ops in ``test_gpu_epilogue.py``; every op here is row by row, so equality
+is the whole contract. Rows of zeros, negative zeros and large values are among the inputs.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from miattn import PagedPool
+from miattn.qwen3 import rope_table
+
+pytestmark = pytest.mark.gpu
+
+
+def _bits(t):
+    return t.view(torch.int16)
+
+
+def _values(g, *shape, dtype, scale=1.0):
+    t = (torch.randn(*shape, generator=g) * scale).to(dtype)
+    flat = t.view(-1)
+    flat[::97] = 0.0
+    flat[5::193] = -0.0
+    t[shape[0] // 2] = 0.0   # a whole row of zeros
+    t[-1] *= 200.0
+    return t.cuda()
+
+
+# rows x heads x D from 2^20 values on take the 16-byte kernel; 1024 rows on, one workgroup per row
+@pytest.mark.parametrize("rows,heads,rotary", [
+    (260, (16, 8, 128), 128), (1025, (16, 8, 128), 64), (1030, (8, 2, 256), 64), (342, (8, 2, 256), 256),
+    (1100, (4, 2, 256), 128), (900, (7, 7, 64), 64), (1300, (12, 3, 64), 64),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("zero_centred", [False, True], ids=["qwen3-norm", "qwen35-norm"])
+def test_epilogue_of_many_rows_is_the_small_batches(rows, heads, rotary, dtype, zero_centred):
+    H, H_kv, D = heads
+    g = torch.Generator().manual_seed(rows)
+    width = (H + 2 * H_kv) * D
+    assert rows * width >= 1 << 20
+    pad = 8 if rotary == 64 else 0  # a longer row stride, still 16-byte rows
+    qkv = _values(g, rows, width + pad, dtype=dtype, scale=2.0)[:, :width]
+    qn, kn = ((1.0 + 0.1 * torch.randn(D, generator=g)).to(dtype).cuda() for _ in range(2))
+    cos, sin = rope_table(rotary, 1e6, 2048, "cuda", dtype)
+    pos = torch.randint(0, 2048, (rows,), generator=g).cuda()
+    n_blocks = rows // 16 + 2
+    slots = torch.randperm(n_blocks * 16, generator=g)[:rows].to(torch.int32 if pad else torch.int64).cuda()
+    slots[3] = -1                 # nothing to write
+    slots[rows - 2] = n_blocks * 16  # refused: past the pool
+    pos[7] = 2048                 # refused: past the RoPE table
+    got, want = {}, {}
+    for out, step in ((got, rows), (want, 50)):
+        assert step == rows or step * width < 1 << 20
+        pool = PagedPool(1, n_blocks, 16, H_kv, D, dtype=dtype, device="cuda", n_head=H)
+        k, v = (torch.full((rows, H_kv, D), 9.0, dtype=dtype, device="cuda") for _ in range(2))
+        q = []
+        for a in range(0, rows, step):
+            b = min(rows, a + step)
+            q.append(pool.write_qk_norm_rope(0, slots[a:b], qkv[a:b], qn, kn, cos, sin, pos[a:b], 1e-6, k_out=k[a:b],
+                                             v_out=v[a:b], rotary_dim=rotary, zero_centred_norm=zero_centred))
+        torch.cuda.synchronize()
+        out.update(q=torch.cat(q), k=k, v=v, keys=pool.keys[0], values=pool.values[0])
+        with pytest.raises(IndexError):
+            pool.check_writes()
+    for name in got:
+        assert torch.equal(_bits(got[name]), _bits(want[name])), name
+    assert not got["q"][[3, 7, rows - 2]].any() and not got["k"][[3, 7, rows - 2]].any()
