@@ -19,6 +19,7 @@
 // them in split order and rounds once to the activation dtype, the value the projection's
 // own output would hold, before the chain above.
 #include <climits>
+#include <initializer_list>
 #include <type_traits>
 
 #include "common.h"
@@ -189,6 +190,30 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(ProjIn<T, kU> gu, T* __re
   out[row * inter + i] = from_f32<T>(rnd<T>(sg * u));
 }
 
+// The same over a T projection with 16-byte accesses (inter % 8 == 0, 16-bit types). Bound by
+// memory (rows x inter x 3 values); the projection is read once, nontemporal. Measured (bf16,
+// inter 3072, graph replay) against the kernel above, one 2-byte element per lane: 8192 rows 59.0
+// -> 29.9 us (151 MB, 5.0 TB/s; a large copy reaches 5.1), 4311 rows 31.8 -> 17.7, 512 rows 4.0 either way.
+template <typename T>
+__global__ __launch_bounds__(256) void silu_mul_vec_kernel(const T* __restrict__ gu, T* __restrict__ out, int inter) {
+  constexpr int E = 8;
+  const int64_t row = blockIdx.y;
+  const int i = (blockIdx.x * blockDim.x + threadIdx.x) * E;
+  if (i >= inter) return;
+  const uint4 gr = load16_nt(gu + row * 2 * inter + i);
+  const uint4 ur = load16_nt(gu + row * 2 * inter + inter + i);
+  float o[E];
+#pragma unroll
+  for (int k = 0; k < E; ++k) {
+    const float g = Vec16<T>::get(gr, k);
+    o[k] = g / (1.0f + expf(-g));
+  }
+  rt8<T>(o);
+#pragma unroll
+  for (int k = 0; k < E; ++k) o[k] *= Vec16<T>::get(ur, k);
+  store16(out + row * inter + i, rt8<T>(o));
+}
+
 template <typename T, int PER>
 int launch_norm_per(const void* x, const void* delta, int delta_parts, const void* w, void* x_out, void* h_out,
                     int rows, int cols, float eps, hipStream_t s) {
@@ -215,6 +240,12 @@ int launch_norm_per(const void* x, const void* delta, int delta_parts, const voi
   return launch_status("mi_add_rms_norm");
 }
 
+bool aligned16(std::initializer_list<const void*> ps) {
+  uintptr_t all = 0;
+  for (const void* p : ps) all |= reinterpret_cast<uintptr_t>(p);
+  return all % 16 == 0;
+}
+
 template <typename T>
 int launch_norm(const void* x, const void* delta, int delta_parts, const void* w, void* x_out, void* h_out,
                 int rows, int cols, float eps, hipStream_t s) {
@@ -223,8 +254,19 @@ int launch_norm(const void* x, const void* delta, int delta_parts, const void* w
   return launch_norm_per<T, 16>(x, delta, delta_parts, w, x_out, h_out, rows, cols, eps, s);
 }
 
+// Outputs from which the 16-byte silu kernel runs (inter 3072: 32 rows 2.06 against 2.16 us, 128
+// rows 2.24 either way, 256 rows 2.74 against 2.70).
+constexpr int64_t kVecValues = 1 << 19;
+
 template <typename T>
 int launch_silu(const void* gu, int gu_parts, void* out, int rows, int inter, hipStream_t s) {
+  if constexpr (sizeof(T) == 2) {
+    if (gu_parts == 0 && int64_t(rows) * inter >= kVecValues && inter % 8 == 0 && aligned16({gu, out})) {
+      hipLaunchKernelGGL((silu_mul_vec_kernel<T>), dim3((inter / 8 + 255) / 256, rows), dim3(256), 0, s,
+                         static_cast<const T*>(gu), static_cast<T*>(out), inter);
+      return launch_status("mi_silu_mul");
+    }
+  }
   const dim3 grid((inter + 255) / 256, rows);
   const int64_t plane = int64_t(rows) * 2 * inter;
   auto go = [&](auto unroll) {

@@ -11,7 +11,7 @@ import pytest
 import torch
 
 from miattn import PagedPool
-from miattn.qwen3 import rope_table
+from miattn.qwen3 import rope_table, silu_mul
 
 pytestmark = pytest.mark.gpu
 
@@ -69,3 +69,18 @@ def test_epilogue_of_many_rows_is_the_small_batches(rows, heads, rotary, dtype, 
     for name in got:
         assert torch.equal(_bits(got[name]), _bits(want[name])), name
     assert not got["q"][[3, 7, rows - 2]].any() and not got["k"][[3, 7, rows - 2]].any()
+
+
+@pytest.mark.parametrize("rows,inter", [(512, 1024), (1001, 3072), (700, 1000), (600, 1004), (65537 // 8, 72)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_silu_mul_of_many_rows_is_the_small_batches(rows, inter, dtype):
+    g = torch.Generator().manual_seed(rows)
+    assert rows * inter >= 1 << 19
+    gu = _values(g, rows, 2 * inter, dtype=dtype, scale=3.0)
+    gu[0, :6] = torch.tensor([float("inf"), -float("inf"), -88.0, -90.0, 90.0, -100.0], dtype=dtype)
+    a = silu_mul(gu)
+    step = max(1, (1 << 18) // inter)
+    b = torch.cat([silu_mul(gu[i:i + step]) for i in range(0, rows, step)])
+    torch.cuda.synchronize()
+    nan = torch.isnan(b)
+    assert torch.equal(nan, torch.isnan(a)) and torch.equal(_bits(a)[~nan], _bits(b)[~nan])
