@@ -124,6 +124,76 @@ __global__ __launch_bounds__(kNormThreads) void add_rms_norm_kernel(
   norm_row<T, PER>(s, wv, cols, eps, x_row, h_out + row * cols);
 }
 
+// The same over T inputs (no partial sums) for many rows: one wave per row with 16-byte
+// accesses, no barrier, four rows per workgroup. For cols a multiple of 512 (NI x 512) and
+// 16-bit types. Bound by memory (rows x cols x 4 values with the add).
+//
+// Bit-equal to the kernel above: its thread t sums the squares of elements t, t + 256, ... in
+// that order, its waves (t = 64 w + l) run the 64-lane butterfly over l and their sums are
+// added in wave order. Here lane L's i-th piece holds elements 512 i + 8 L + k, so t = 8 (L mod
+// 32) + k and the elements of one t alternate between lanes L and L + 32; l is (k, lane bits
+// 0-2) -- the in-lane tree over k, then an 8-lane butterfly -- and w is lane bits 3-4.
+template <typename T, bool kAdd, int NI>
+__global__ __launch_bounds__(256) void add_rms_norm_wave_kernel(const T* x, const T* __restrict__ delta,
+                                                                const T* __restrict__ w, T* x_out,
+                                                                T* __restrict__ h_out, int rows, float eps) {
+  constexpr int E = 8, cols = NI * 512;
+  const int lane = threadIdx.x & 63;
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= rows) return;  // wave-uniform, no barrier follows
+  const int64_t base = int64_t(row) * cols + lane * E;
+  uint4 xr[NI], dr[NI], wr[NI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    xr[i] = load16(x + base + i * 512);
+    if constexpr (kAdd) dr[i] = load16(delta + base + i * 512);
+    wr[i] = load16(w + lane * E + i * 512);
+  }
+  float acc[E];
+#pragma unroll
+  for (int k = 0; k < E; ++k) acc[k] = 0.0f;
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    float s[E], sq[E];
+#pragma unroll
+    for (int k = 0; k < E; ++k) {
+      s[k] = Vec16<T>::get(xr[i], k);
+      if constexpr (kAdd) s[k] += Vec16<T>::get(dr[i], k);
+    }
+    if constexpr (kAdd) xr[i] = rt8<T>(s);
+#pragma unroll
+    for (int k = 0; k < E; ++k) sq[k] = s[k] * s[k];
+    rt8<T>(sq);
+#pragma unroll
+    for (int k = 0; k < E; ++k) {
+      // [0]: the low half's value in every lane, [1]: the high half's
+      const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(sq[k]), __float_as_uint(sq[k]), false, false);
+      acc[k] = (acc[k] + __uint_as_float(both[0])) + __uint_as_float(both[1]);
+    }
+  }
+  const float part = group_allreduce<8, SumOp>(((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7])));
+  const float part8 = dpp<kDppRowRor8>(part);
+  const float even = (lane & 8) ? part8 : part, odd = (lane & 8) ? part : part8;
+  const float even16 = swap16(even), odd16 = swap16(odd);
+  const bool hi = lane & 16;
+  const float total = (((hi ? even16 : even) + (hi ? odd16 : odd)) + (hi ? even : even16)) + (hi ? odd : odd16);
+  const float ms = rnd<T>(total * (1.0f / float(cols)));
+  const float rms = rnd<T>(sqrtf(rnd<T>(ms + eps)));
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    float h[E];
+#pragma unroll
+    for (int k = 0; k < E; ++k) h[k] = Vec16<T>::get(xr[i], k);
+    div_rt8<T>(h, rms);
+#pragma unroll
+    for (int k = 0; k < E; ++k) h[k] *= Vec16<T>::get(wr[i], k);
+    if constexpr (kAdd) {
+      if (x_out != nullptr) store16(x_out + base + i * 512, xr[i]);
+    }
+    store16(h_out + base + i * 512, rt8<T>(h));
+  }
+}
+
 // Start of a captured decode step, one workgroup per row: seqlen = pos + 1, the row's write
 // slot table[pos / bs] * bs + pos % bs (reference model/paged.py:499-501), x = embed[token]
 // (the embedding lookup) and h = rmsnorm(x) * w (layer 0's input norm).
@@ -240,6 +310,10 @@ int launch_norm_per(const void* x, const void* delta, int delta_parts, const voi
   return launch_status("mi_add_rms_norm");
 }
 
+// Rows from which the wave-per-row kernel runs (a quarter of the workgroups: at 128 rows one
+// barrier in 128 workgroups is as fast, 2.8 us, and below that faster).
+constexpr int kWaveRows = 256;
+
 bool aligned16(std::initializer_list<const void*> ps) {
   uintptr_t all = 0;
   for (const void* p : ps) all |= reinterpret_cast<uintptr_t>(p);
@@ -249,6 +323,31 @@ bool aligned16(std::initializer_list<const void*> ps) {
 template <typename T>
 int launch_norm(const void* x, const void* delta, int delta_parts, const void* w, void* x_out, void* h_out,
                 int rows, int cols, float eps, hipStream_t s) {
+  if constexpr (sizeof(T) == 2) {
+    if (rows >= kWaveRows && cols % 512 == 0 && (delta == nullptr || delta_parts == 0) &&
+        aligned16({x, delta, w, x_out, h_out})) {
+      auto go = [&](auto add, auto ni) {
+        hipLaunchKernelGGL((add_rms_norm_wave_kernel<T, decltype(add)::value, decltype(ni)::value>),
+                           dim3((rows + 3) / 4), dim3(256), 0, s, static_cast<const T*>(x),
+                           static_cast<const T*>(delta), static_cast<const T*>(w), static_cast<T*>(x_out),
+                           static_cast<T*>(h_out), rows, eps);
+      };
+      auto by_add = [&](auto ni) {
+        if (delta != nullptr) go(std::true_type{}, ni); else go(std::false_type{}, ni);
+      };
+      switch (cols / 512) {
+        case 1: by_add(std::integral_constant<int, 1>{}); break;
+        case 2: by_add(std::integral_constant<int, 2>{}); break;
+        case 3: by_add(std::integral_constant<int, 3>{}); break;
+        case 4: by_add(std::integral_constant<int, 4>{}); break;
+        case 5: by_add(std::integral_constant<int, 5>{}); break;
+        case 6: by_add(std::integral_constant<int, 6>{}); break;
+        case 7: by_add(std::integral_constant<int, 7>{}); break;
+        default: by_add(std::integral_constant<int, 8>{}); break;  // cols <= 4096
+      }
+      return launch_status("mi_add_rms_norm");
+    }
+  }
   if (cols <= 4 * kNormThreads) return launch_norm_per<T, 4>(x, delta, delta_parts, w, x_out, h_out, rows, cols, eps, s);
   if (cols <= 8 * kNormThreads) return launch_norm_per<T, 8>(x, delta, delta_parts, w, x_out, h_out, rows, cols, eps, s);
   return launch_norm_per<T, 16>(x, delta, delta_parts, w, x_out, h_out, rows, cols, eps, s);

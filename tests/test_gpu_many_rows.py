@@ -11,7 +11,7 @@ import pytest
 import torch
 
 from miattn import PagedPool
-from miattn.qwen3 import rope_table, silu_mul
+from miattn.qwen3 import add_rms_norm, rope_table, silu_mul
 
 pytestmark = pytest.mark.gpu
 
@@ -69,6 +69,25 @@ def test_epilogue_of_many_rows_is_the_small_batches(rows, heads, rotary, dtype, 
     for name in got:
         assert torch.equal(_bits(got[name]), _bits(want[name])), name
     assert not got["q"][[3, 7, rows - 2]].any() and not got["k"][[3, 7, rows - 2]].any()
+
+
+@pytest.mark.parametrize("rows,cols", [(256, 512), (259, 1024), (1001, 1536), (300, 2560), (257, 4096)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("with_delta", [True, False])
+def test_add_rms_norm_of_many_rows_is_the_small_batches(rows, cols, dtype, with_delta):
+    g = torch.Generator().manual_seed(rows + cols)
+    x = _values(g, rows, cols, dtype=dtype)
+    d = _values(g, rows, cols, dtype=dtype, scale=0.5) if with_delta else None
+    w = (1.0 + 0.1 * torch.randn(cols, generator=g)).to(dtype).cuda()
+    for eps in (1e-6, 0.0):  # eps 0: a row of zeros divides by zero, NaN in both
+        xa, xb = x.clone(), x.clone()
+        _, ha = add_rms_norm(xa, d, w, eps)
+        hb = torch.cat([add_rms_norm(xb[a:a + 100], None if d is None else d[a:a + 100], w, eps)[1]
+                        for a in range(0, rows, 100)])
+        torch.cuda.synchronize()
+        nan = torch.isnan(hb)
+        assert torch.equal(_bits(xa), _bits(xb)) and torch.equal(nan, torch.isnan(ha))
+        assert torch.equal(_bits(ha)[~nan], _bits(hb)[~nan]) and nan.any().item() == (eps == 0.0)
 
 
 @pytest.mark.parametrize("rows,inter", [(512, 1024), (1001, 3072), (700, 1000), (600, 1004), (65537 // 8, 72)])
