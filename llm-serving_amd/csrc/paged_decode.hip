@@ -13,8 +13,9 @@
 //     served by the lanes holding that KV head, so each K/V byte is read once (the
 //     reference launches one program per query head and relies on the cache, :33-36);
 //   * token-balanced split-K, planned on the device: every workgroup reads the row lengths,
-//     sets chunk = ceil(sum(seqlen) / kTargetSplits) (rounded to a batch) and maps its
-//     index to (row, split) through a prefix sum of the rows' split counts. Every split
+//     sets the tokens per split so that the splits of all rows fit the workgroups aimed for
+//     (plan_chunk) and maps its index to (row, split) through a prefix sum of the rows'
+//     split counts. Every split
 //     therefore carries the same number of tokens however ragged the batch is, the grid
 //     (kTargetSplits + B workgroups, sized without a host read of seqlen) fills the 256
 //     CUs, and long rows (config 4) and short ones cost the same per token;
@@ -35,6 +36,7 @@
 //   * K/V are read with the nontemporal hint: each byte is used once, and keeping it out
 //     of L2 lifted config 2 from 43.0 to 39.4 us and config 4 from 5.3 to 6.0 TB/s.
 // HBM-bound: per (token, KV head) the kernel reads 2 * D * esize bytes of K+V.
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -44,7 +46,7 @@ namespace miattn {
 namespace {
 
 struct DecodeArgs {
-  int B, H, H_kv, G, kvb_log2, n_hchunks, bs_log2, max_blocks, target, slots;
+  int B, H, H_kv, G, kvb_log2, n_hchunks, bs_log2, max_blocks, target, target_log2, half, half_log2, half_max, slots;
   int64_t qs0, qs1, ks0, ks1, ks2, vs0, vs1, vs2, os0, os1, bts0;
   float scale_log2;
 };
@@ -76,7 +78,8 @@ struct FusedArgs {
 constexpr int kThreads = MIATTN_DECODE_THREADS;
 constexpr int kWaves = kThreads / 64;
 
-// Workgroups a launch aims for: 2 per CU of the 256-CU MI355X, all resident at once.
+// Workgroups a launch aims for at most: 2 per CU of the 256-CU MI355X, all resident at once
+// (make_plan and plan_chunk choose between this and half of it).
 #ifndef MIATTN_DECODE_TARGET_SPLITS
 #define MIATTN_DECODE_TARGET_SPLITS 512
 #endif
@@ -160,13 +163,6 @@ __device__ __forceinline__ int clamp_len(int len, int capacity) {
   return len > 0 ? len : 0;
 }
 
-// Tokens per split for a batch holding `total` tokens (identical in both launches).
-__device__ __forceinline__ int split_chunk(int total, int batch, int target) {
-  int chunk = (total + target - 1) / target;
-  chunk = (chunk + batch - 1) / batch * batch;
-  return chunk > batch ? chunk : batch;
-}
-
 // Inclusive prefix sum over the 64 lanes of a wave, in DPP moves (no LDS round trips):
 // shifts by 1, 2, 4 and 8 inside each row of 16 lanes (lanes shifted in from outside the
 // row read 0), then lane 15 of rows 0 and 2 added into rows 1 and 3, and lane 31 into rows
@@ -181,6 +177,57 @@ __device__ __forceinline__ int wave_inclusive_scan(int v) {
   return v;
 }
 
+// Floors of the split size, in tokens. A split of one 8-token batch is all latency and a row of
+// many of them is several round trips of the merge, so past kTinyTokens in the batch a split
+// holds at least kSplitFloor tokens, and at or below it a row of more than 32 such batches (the
+// splits the merge folds per round trip) at least kSplitFloorLongRow. Measured (H 16 / H_kv 8 / D
+// 128, us per layer, splits of 8 / 16 / 24 / 32 tokens): 4 rows of 429 tokens in all 7.2 / 7.6 / 8.7 /
+// 9.1, one row of 300 7.8 / 7.4 / 8.5 / 8.9, one row of 2048 14.9 / 10.9 / 10.8 / 10.3, 8 rows of 512
+// 12.4 / 9.7 / 9.8 / 9.9. Of the sizes between 16 and 32 above kTinyTokens, 24 is the one whose fp32
+// summation order keeps the greedy tokens as close to the CPU path's as they were.
+constexpr int kTinyTokens = 1024;
+constexpr int kSplitFloor = 24;
+constexpr int kSplitFloorLongRow = 16;
+constexpr int kFitSteps = 16;
+
+// Tokens per split of this batch: the splits of all rows (partial ones at the rows' ends counted)
+// fit the workgroups aimed for. A chunk of ceil(total / target) alone overflowed them by up to
+// one split per row, and the CUs that took a workgroup more than the others finished last (32
+// rows of 128-2048 tokens 43.9 -> 36.9 us, 64 rows 62 -> 52 us; batches that happened to fit are
+// as before). Also returns the split count of this lane's row of the first 64 and its inclusive
+// scan. Not fitted: batches past 64 rows (their lengths are not all in registers) and of more
+// than a quarter as many rows as workgroups (their partial splits are no small excess).
+__device__ __forceinline__ int plan_chunk(int len_first, int total, const DecodeArgs& a, int batch, int& n, int& incl) {
+  // ceil(total / t) in whole batches (a batch is a power of two)
+  auto chunk_for = [&](int t, int log2) {
+    const uint32_t x = uint32_t(total) + uint32_t(t) - 1u;
+    const uint32_t c = log2 >= 0 ? x >> log2 : x / uint32_t(t);
+    return int((c + batch - 1) & -batch);
+  };
+  int t = a.target;
+  int chunk = chunk_for(t, a.target_log2);
+  if (a.half > 0) {
+    const int c = chunk_for(a.half, a.half_log2);
+    if (c <= a.half_max) {
+      t = a.half;
+      const int least = total > kTinyTokens ? kSplitFloor : __any(len_first > 32 * batch) ? kSplitFloorLongRow : 0;
+      chunk = max(c, (least + batch - 1) & -batch);
+    }
+  }
+  chunk = max(chunk, batch);
+  for (int i = 0;; ++i) {
+    // n = ceil(len / chunk), exact: the quotient is at most a few hundred, so the product is off
+    // by less than one either way
+    const uint32_t x = uint32_t(len_first) + uint32_t(chunk) - 1u;
+    n = int(float(x) * __builtin_amdgcn_rcpf(float(chunk)));
+    const int r = int(x - uint32_t(n) * uint32_t(chunk));
+    n += r < 0 ? -1 : r >= chunk ? 1 : 0;
+    incl = wave_inclusive_scan(n);
+    if (i == kFitSteps || a.B > 64 || 4 * a.B > t || __builtin_amdgcn_readlane(incl, 63) <= t) return chunk;
+    chunk += batch;
+  }
+}
+
 // This workgroup's piece of the token-balanced split: row b, split index within the row,
 // the row's split count and the global index of its first split. Every wave derives it on
 // its own from the row lengths (same inputs, same answer), so planning needs no LDS and no
@@ -188,8 +235,9 @@ __device__ __forceinline__ int wave_inclusive_scan(int v) {
 struct SplitInfo {
   int b, split, n_split, first, chunk, len;
 };
-__device__ __forceinline__ bool plan_split(const int32_t* __restrict__ seqlen, int B, int capacity,
-                                           int batch, int target, int w, SplitInfo& si) {
+__device__ __forceinline__ bool plan_split(const int32_t* __restrict__ seqlen, int capacity, int batch,
+                                           const DecodeArgs& a, int w, SplitInfo& si) {
+  const int B = a.B;
   const int lane = __lane_id();
   // the first 64 rows' lengths are loaded once and serve both passes (one round trip for
   // batches of up to 64 rows)
@@ -200,13 +248,11 @@ __device__ __forceinline__ bool plan_split(const int32_t* __restrict__ seqlen, i
     const int len = row < B ? clamp_len(seqlen[row], capacity) : 0;
     total += __builtin_amdgcn_readlane(wave_inclusive_scan(len), 63);
   }
-  const int chunk = split_chunk(total, batch, target);
+  int n, incl;
+  const int chunk = plan_chunk(len_first, total, a, batch, n, incl);
+  int len = len_first;
   int base = 0;  // splits of the rows before this block of 64
-  for (int r0 = 0; r0 < B; r0 += 64) {
-    const int row = r0 + lane;
-    const int len = r0 == 0 ? len_first : row < B ? clamp_len(seqlen[row], capacity) : 0;
-    const int n = (len + chunk - 1) / chunk;
-    const int incl = wave_inclusive_scan(n);
+  for (int r0 = 0;;) {
     const uint64_t owner = __ballot(w >= base + incl - n && w < base + incl);
     if (owner != 0) {
       const int o = __ffsll(static_cast<unsigned long long>(owner)) - 1;
@@ -219,9 +265,14 @@ __device__ __forceinline__ bool plan_split(const int32_t* __restrict__ seqlen, i
       si.len = __builtin_amdgcn_readlane(len, o);  // the row's length, already in lane o
       return true;
     }
+    r0 += 64;
+    if (r0 >= B) return false;  // w is past the last split
     base += __builtin_amdgcn_readlane(incl, 63);
+    const int row = r0 + lane;
+    len = row < B ? clamp_len(seqlen[row], capacity) : 0;
+    n = (len + chunk - 1) / chunk;
+    incl = wave_inclusive_scan(n);
   }
-  return false;  // w is past the last split
 }
 
 // UP ("uniform pages"): every lane of a wave reads the same token of a workgroup-wide load
@@ -247,7 +298,7 @@ __global__ __launch_bounds__(kThreads) void paged_decode_kernel(
 
   // ---- device-side split plan: total tokens -> chunk -> this workgroup's (row, split)
   SplitInfo si;
-  if (!plan_split(seqlen, a.B, capacity, batch, a.target, blockIdx.x, si)) return;  // uniform
+  if (!plan_split(seqlen, capacity, batch, a, blockIdx.x, si)) return;  // uniform
   const int b = si.b, split = si.split, n_split_b = si.n_split, first_slot = si.first;
   const int chunk = si.chunk;
   const int len = si.len;
@@ -724,7 +775,7 @@ int lowbit(int x) { return x & -x; }
 
 // Launch geometry, computed identically by the workspace query and the launcher.
 struct Plan {
-  int GB, n_hchunks, KVB, kvb_log2, n_groups, NR, TPL, U, target, slots;
+  int GB, n_hchunks, KVB, kvb_log2, n_groups, NR, TPL, U, target, half, half_max, slots;
   size_t rows_bytes, ml_bytes, acc_bytes;
   size_t smem_bytes;
 };
@@ -756,6 +807,15 @@ Plan make_plan(int B, int H, int H_kv, int D, int block_size, int max_blocks, in
   // total / target, and each row adds at most one partial split.
   const int cols = p.n_groups * p.n_hchunks;
   p.target = kTargetSplits / cols > 0 ? kTargetSplits / cols : 1;
+  // Half of them (one 4-wave workgroup per CU) for splits of up to half_max tokens. With 1 or 2 query
+  // heads per lane one workgroup streams as fast as two, and half the splits leave half the
+  // merging (16 rows of 256: 11.6 -> 9.9 us per layer, 8 of 2048 19.4 -> 17.1, 32 of 8192 175.5 ->
+  // 172.4). With more heads per lane a wave's arithmetic shows, and two workgroups hide each
+  // other's from 128 tokens on (H 8 / H_kv 2 / D 256, 35229 tokens: 22.3 against 23.1 us); split
+  // over several workgroup columns it shows from the start (H 32 / H_kv 4 / D 128, 8 rows of 512:
+  // 12.5 against 13.3 us).
+  p.half = p.n_hchunks == 1 && 4 * B <= p.target / 2 ? p.target / 2 : 0;
+  p.half_max = p.GB <= 2 ? INT32_MAX : 128;
   p.slots = p.target + B;
   // parked row states of the tsub > 0 rows: (m, l) pairs padded to 16 bytes, then acc
   const size_t parked = size_t(p.TPL - 1) * p.KVB * p.GB;
@@ -920,7 +980,9 @@ int paged_decode_entry(const void* q, const void* k_cache, const void* v_cache, 
   DecodeArgs a;
   a.B = B; a.H = H; a.H_kv = H_kv; a.G = H / H_kv; a.kvb_log2 = p.kvb_log2;
   a.n_hchunks = p.n_hchunks; a.bs_log2 = bs_log2;
-  a.max_blocks = max_blocks; a.target = p.target; a.slots = p.slots;
+  a.max_blocks = max_blocks; a.target = p.target; a.target_log2 = ilog2_exact(p.target);
+  a.half = p.half; a.half_log2 = p.half > 0 ? ilog2_exact(p.half) : -1; a.half_max = p.half_max;
+  a.slots = p.slots;
   a.qs0 = st[0]; a.qs1 = st[1];
   a.ks0 = st[3]; a.ks1 = st[4]; a.ks2 = st[5];
   a.vs0 = st[7]; a.vs1 = st[8]; a.vs2 = st[9];

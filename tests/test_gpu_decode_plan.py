@@ -1,0 +1,83 @@
+"""The decode's device-side split plan at the sizes where it changes its mind: the batch's
+token total around the point from which splits have a floor, rows around 32 batches, ragged
+batches whose partial splits overflow the workgroups aimed for (the split size is then fitted),
+64 and 65 rows (fitted or not), and head layouts with one or several workgroup columns and
+with 4 query heads per lane around 128-token splits.
+
+Each result is held to the fp32 gather oracle within 2e-2 and, beyond its own 16-bit rounding
+(2^-8 relative for bf16), within 1e-3, the bars of ``test_gpu_decode.py``: a plan that drops,
+repeats or misplaces a split misses them by orders of magnitude. The plan must not depend on
+anything but the row lengths: the same rows through a wider table give the same bits.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from miattn import paged_decode
+from oracle.decode import reference_paged_decode
+
+pytestmark = pytest.mark.gpu
+
+BS = 16
+
+
+def _build(lengths, H, H_kv, D, dtype, seed):
+    g = torch.Generator().manual_seed(seed)
+    pages = [-(-n // BS) for n in lengths]
+    n_blocks = sum(pages) + 3
+    k, v = (torch.randn(n_blocks, BS, H_kv, D, generator=g).to(dtype) for _ in range(2))
+    q = torch.randn(len(lengths), H, D, generator=g).to(dtype)
+    perm = torch.randperm(n_blocks, generator=g).to(torch.int32)
+    table = torch.zeros(len(lengths), max(max(pages), 1), dtype=torch.int32)
+    at = 0
+    for r, n in enumerate(pages):
+        table[r, :n] = perm[at:at + n]
+        at += n
+    return q, k, v, table, torch.tensor(lengths, dtype=torch.int32)
+
+
+def _ragged(n, lo, hi, seed):
+    return torch.randint(lo, hi + 1, (n,), generator=torch.Generator().manual_seed(seed)).tolist()
+
+
+QWEN3 = (16, 8, 128)
+CASES = [
+    pytest.param([1023], QWEN3, id="one-row-1023"),
+    pytest.param([1024], QWEN3, id="one-row-1024"),
+    pytest.param([1025], QWEN3, id="one-row-1025"),
+    pytest.param([256, 100], QWEN3, id="32-batches"),
+    pytest.param([257, 100], QWEN3, id="past-32-batches"),
+    pytest.param([512, 500, 12], QWEN3, id="total-1024"),
+    pytest.param([512, 501, 12], QWEN3, id="total-1025"),
+    pytest.param(_ragged(32, 128, 2048, 5), QWEN3, id="ragged-32"),
+    pytest.param(_ragged(64, 1, 700, 6), QWEN3, id="ragged-64"),
+    pytest.param(_ragged(65, 1, 700, 7), QWEN3, id="ragged-65"),
+    pytest.param([0] * 20 + [1] * 40 + [3000, 0, 2500, 1], QWEN3, id="mostly-short"),
+    pytest.param([8192] + [17] * 31, QWEN3, id="one-long"),
+    pytest.param(_ragged(33, 1, 900, 8), (32, 16, 128), id="two-columns"),
+    pytest.param(_ragged(16, 100, 1500, 9), (32, 4, 128), id="head-chunks"),
+    pytest.param(_ragged(30, 1, 1200, 10), (16, 16, 64), id="d64"),
+    pytest.param([2048] * 16, (8, 2, 256), id="4-heads-128-tokens"),
+    pytest.param([2048] * 16 + [9], (8, 2, 256), id="4-heads-past-128-tokens"),
+    pytest.param(_ragged(16, 128, 2048, 11), (8, 2, 256), id="4-heads-ragged"),
+    pytest.param(_ragged(9, 1, 300, 12), (10, 5, 128), id="five-columns"),
+]
+
+
+@pytest.mark.parametrize("lengths,heads", CASES)
+def test_split_plan_edges(lengths, heads, cuda):
+    H, H_kv, D = heads
+    q, k, v, table, seqlen = _build(lengths, H, H_kv, D, torch.bfloat16, seed=len(lengths))
+    want = reference_paged_decode(q, k, v, table, seqlen, out_dtype=torch.float32)
+    dev = [t.to(cuda) for t in (q, k, v, table, seqlen)]
+    got = paged_decode(*dev)
+    wide = torch.cat([dev[3], torch.full((len(lengths), 9), -999, dtype=torch.int32, device=cuda)], 1)
+    again = paged_decode(dev[0], dev[1], dev[2], wide, dev[4])
+    torch.cuda.synchronize()
+    assert torch.equal(got, again)
+    diff = (got.cpu().float() - want).abs()
+    assert diff.max().item() <= 2e-2
+    assert (diff - want.abs() * 2.0 ** -8).max().item() <= 1e-3
+    assert not got[seqlen == 0].any()
