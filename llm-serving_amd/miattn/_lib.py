@@ -168,9 +168,16 @@ def dtype_code(dtype: torch.dtype) -> int:
         raise ValueError(f"dtype must be fp16, bf16 or fp32, got {dtype}") from None
 
 
+#: torch's current stream of a device index as a raw handle: 0.06 us, against 2 us for the
+#: ``torch.cuda.Stream`` object, which every launch paid for and threw away
+_RAW_STREAM = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def current_stream(device: torch.device) -> int:
     """Raw ``hipStream_t`` of torch's current stream on ``device``."""
-    return torch.cuda.current_stream(device).cuda_stream
+    if _RAW_STREAM is None or device.index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return _RAW_STREAM(device.index)
 
 
 def last_error() -> str:

@@ -263,7 +263,7 @@ class PagedDecodePlan:
     """
 
     __slots__ = ("n_layer", "geometry", "q_signature", "_k_ptrs", "_v_ptrs", "_pools",
-                 "_table", "_seqlen", "_strides", "_scale", "_ws", "_ws_bytes")
+                 "_table", "_seqlen", "_strides", "_scale", "_ws", "_ws_bytes", "_frozen")
 
     def __init__(self, q, k_caches, v_caches, block_table, seqlen, *, scale=None) -> None:
         _require_backend()
@@ -291,6 +291,9 @@ class PagedDecodePlan:
         self._scale = float(1.0 / math.sqrt(g.head_dim) if scale is None else scale)
         self._ws_bytes = _workspace_bytes(g, q.dtype)
         self._ws = torch.empty(self._ws_bytes, dtype=torch.uint8, device=q.device) if self._ws_bytes else None
+        # the launch arguments after ``out`` that no run changes (the plan owns the workspace)
+        self._frozen = (*g.dims(), self._strides, self._scale, _lib.dtype_code(q.dtype),
+                        None if self._ws is None else self._ws.data_ptr(), self._ws_bytes)
 
     def run(self, layer: int, q):
         """Launch one layer; ``q`` must have the layout the plan was built with."""
@@ -305,11 +308,11 @@ class PagedDecodePlan:
             )
         out = torch.empty_like(q)
         layer = int(layer)
-        _launch(self.geometry, q, self._k_ptrs[layer], self._v_ptrs[layer], self._table.data_ptr(),
-                self._seqlen.data_ptr(), out, self._strides, self._scale,
-                None if self._ws is None else self._ws.data_ptr(), self._ws_bytes, "paged_decode_plan.run")
+        rc = _lib.lib.mi_paged_decode(q.data_ptr(), self._k_ptrs[layer], self._v_ptrs[layer], self._table.data_ptr(),
+                                      self._seqlen.data_ptr(), out.data_ptr(), *self._frozen,
+                                      _lib.current_stream(q.device))
+        _lib.check(rc, "paged_decode_plan.run")
         return out
-
 
     def fused_supported(self, dtype: torch.dtype, rotary_dim: int, zero_centred_norm: bool = False) -> bool:
         """Whether :meth:`run_fused` covers this geometry: head_dim 128, whole-head RoPE, the

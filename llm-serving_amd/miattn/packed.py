@@ -16,8 +16,10 @@ that launch.
 
 from __future__ import annotations
 
+from itertools import chain
 from typing import Sequence
 
+import numpy as np
 import torch
 
 __all__ = ["PackedPrefill", "as_packed_prefill", "PACKED_PREFILL_FLAG"]
@@ -63,8 +65,7 @@ class PackedPrefill:
         if min(b - a for a, b in zip(cu, cu[1:])) <= 0:
             raise ValueError(f"cu_seqlens must be strictly increasing, got {cu}")
         sinks = list(sinks)
-        if len(sinks) != len(cu) - 1:
-            raise ValueError(f"PackedPrefill needs one sink per request ({len(cu) - 1}), got {len(sinks)}")
+        self._check_sinks(cu, sinks)
         total = cu[-1]
         if positions.dim() != 1 or positions.numel() != total:
             raise ValueError(f"positions must be a 1-D tensor of {total} entries, got {tuple(positions.shape)}")
@@ -76,6 +77,50 @@ class PackedPrefill:
             row = max(i for i in range(len(cu) - 1) if cu[i] <= t)
             raise ValueError(f"request {row}: positions must be request-local 0..{cu[row + 1] - cu[row] - 1} "
                              "(a packed layout does not share one increasing position axis)")
+        self._set_up(cu, positions, sinks, backend, torch.tensor(cu[1:], dtype=torch.long, device=positions.device) - 1)
+        self._group = self._one_pool_slots()
+
+    @staticmethod
+    def _check_sinks(cu: list[int], sinks: list) -> None:
+        if len(sinks) != len(cu) - 1:
+            raise ValueError(f"PackedPrefill needs one sink per request ({len(cu) - 1}), got {len(sinks)}")
+
+    @classmethod
+    def upload(cls, prompts: Sequence[Sequence[int]], pool, block_tables, device):
+        """The container of whole prompts written into one paged ``pool``, and their packed tokens.
+        What the group needs on the device -- tokens, request-local positions, slot map, last
+        indices -- is built on the host and uploaded in one copy; nothing is read back, so the
+        host does not wait for work already queued."""
+        from .paged import PagedWriteSink
+
+        lengths = [len(p) for p in prompts]
+        cu = [0]
+        for n in lengths:
+            cu.append(cu[-1] + n)
+        tables = [list(t) for t, _ in zip(block_tables, lengths)]
+        for t, n in zip(tables, lengths):
+            pool._check_block_ids(t, pool._blocks_for(0, n))
+        if len(cu) < 2:
+            raise ValueError("PackedPrefill needs at least one request (cu_seqlens length >= 2)")
+        if min(lengths) <= 0:
+            raise ValueError(f"cu_seqlens must be strictly increasing, got {cu}")
+        cls._check_sinks(cu, tables)  # one table per prompt
+        total, bs = cu[-1], pool.block_size
+        host = np.empty(3 * total + len(lengths), dtype=np.int64)
+        host[:total] = np.fromiter(chain.from_iterable(prompts), dtype=np.int64, count=total)
+        for t, a, b in zip(tables, cu, cu[1:]):
+            at = np.arange(b - a, dtype=np.int64)
+            host[total + a: total + b] = at
+            host[2 * total + a: 2 * total + b] = np.asarray(t, dtype=np.int64)[at // bs] * bs + at % bs
+        host[3 * total:] = np.asarray(cu[1:]) - 1
+        tokens, positions, slots, last = torch.from_numpy(host).to(device).split([total, total, total, len(lengths)])
+        packed = cls.__new__(cls)
+        packed._set_up(cu, positions, [PagedWriteSink(pool, t, n, slots=slots[a: a + n])
+                                       for t, n, a in zip(tables, lengths, cu)], None, last)
+        packed._group = (pool, slots)
+        return packed, tokens
+
+    def _set_up(self, cu: list[int], positions: torch.Tensor, sinks: list, backend, last: torch.Tensor) -> None:
         if backend is None:
             from .varlen import backend_for
 
@@ -84,12 +129,11 @@ class PackedPrefill:
         self.cu_seqlens = cu
         self.positions = positions
         self.sinks = sinks
-        self.total_tokens = total
+        self.total_tokens = cu[-1]
         self.n_seqs = len(sinks)
         self.max_seqlen = max(b - a for a, b in zip(cu, cu[1:]))
         self.rope_len = self.max_seqlen
-        self.last_token_index = torch.tensor(cu[1:], dtype=torch.long, device=positions.device) - 1
-        self._group = self._one_pool_slots()
+        self.last_token_index = last
 
     def _one_pool_slots(self):
         """``(pool, slots)`` when every sink writes one paged pool through a slot map."""

@@ -32,7 +32,7 @@ import torch.nn.functional as F
 from . import _lib
 from .decode import paged_decode_plan
 from .packed import PackedPrefill
-from .paged import PagedKV, PagedPool, PagedWriteSink
+from .paged import PagedKV, PagedPool
 from .rows import Parts, argmax_rows, glu_weight, rows_linear, rows_supported, rows_swiglu, rows_tile_best
 
 __all__ = ["Qwen3Config", "random_weights", "Qwen3", "GraphDecoder"]
@@ -245,14 +245,7 @@ class Qwen3:
         residual add with the next RMSNorm and SiLU * up are one HIP launch each, as in
         decode."""
         c = self.cfg
-        lengths = [len(p) for p in prompts]
-        cu = [0]
-        for n in lengths:
-            cu.append(cu[-1] + n)
-        positions = torch.cat([torch.arange(n) for n in lengths]).to(self.device)
-        sinks = [PagedWriteSink(pool, t, n) for t, n in zip(tables, lengths)]
-        packed = PackedPrefill(cu_seqlens=cu, positions=positions, sinks=sinks)
-        tokens = torch.tensor([t for p in prompts for t in p], dtype=torch.long, device=self.device)
+        packed, tokens = PackedPrefill.upload(prompts, pool, tables, self.device)
         x = F.embedding(tokens, self.w["embed"])  # (T, C), the residual stream (updated in place)
         T = x.shape[0]
         _, h = add_rms_norm(x, None, self.w["l0.ln1"], c.eps)

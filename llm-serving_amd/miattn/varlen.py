@@ -99,9 +99,21 @@ _PACKED = (
 )
 
 
+def _packed_ok(q, k, v) -> bool:
+    """Whether every rule of ``_PACKED`` holds, in one expression (the layer loop's path; the
+    table is walked for its message when this is false)."""
+    if not (isinstance(q, torch.Tensor) and isinstance(k, torch.Tensor) and isinstance(v, torch.Tensor)):
+        return False
+    qs, ks = q.shape, k.shape
+    return (len(qs) == 3 and len(ks) == 3 and ks == v.shape and qs[0] == ks[0] and qs[2] == ks[2] and ks[1] >= 1
+            and qs[1] >= 1 and qs[1] % ks[1] == 0 and q.dtype == k.dtype == v.dtype and q.dtype.is_floating_point
+            and q.device == k.device == v.device)
+
+
 def validate_packed(q, k, v, cu_seqlens, max_seqlen) -> list[int]:
     """Apply the packed layout contract; returns the segment bounds."""
-    enforce(_PACKED, SimpleNamespace(q=q, k=k, v=v))
+    if not _packed_ok(q, k, v):
+        enforce(_PACKED, SimpleNamespace(q=q, k=k, v=v))
     bounds = segment_bounds(cu_seqlens, int(q.shape[0]))
     longest = max(b - a for a, b in zip(bounds, bounds[1:]))
     claimed = as_index(max_seqlen, "max_seqlen")
@@ -151,7 +163,7 @@ class _Schedules:
         self._pinned: dict = {}
 
     def get(self, bounds: list[int], H: int, H_kv: int, D: int, causal: bool, device, kernel: int):
-        key = (tuple(bounds), H, H_kv, D, bool(causal), str(device), kernel)
+        key = (tuple(bounds), H, H_kv, D, bool(causal), device, kernel)
         entry = self._pinned.get(key) or self._lru.get(key)
         if entry is None:
             entry = self._build(bounds, H, H_kv, D, causal, device, kernel)
@@ -207,10 +219,12 @@ def _error_word(device) -> torch.Tensor:
     """The device's prefill error word (one int32, zero when no launch has given up),
     allocated once per device and kept for the life of the process, so a launch recorded in
     a HIP graph keeps a valid address."""
-    key = _device_key(device)
-    word = _ERROR_WORDS.get(key)
+    word = _ERROR_WORDS.get(device)  # a launch's device has an index and is its own key
     if word is None:
-        word = _ERROR_WORDS[key] = torch.zeros(1, dtype=torch.int32, device=key)
+        key = _device_key(device)
+        word = _ERROR_WORDS.get(key)
+        if word is None:
+            word = _ERROR_WORDS[key] = torch.zeros(1, dtype=torch.int32, device=key)
     return word
 
 
