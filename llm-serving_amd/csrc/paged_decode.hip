@@ -810,12 +810,12 @@ Plan make_plan(int B, int H, int H_kv, int D, int block_size, int max_blocks, in
   // Half of them (one 4-wave workgroup per CU) for splits of up to half_max tokens. With 1 or 2 query
   // heads per lane one workgroup streams as fast as two, and half the splits leave half the
   // merging (16 rows of 256: 11.6 -> 9.9 us per layer, 8 of 2048 19.4 -> 17.1, 32 of 8192 175.5 ->
-  // 172.4). With more heads per lane a wave's arithmetic shows, and two workgroups hide each
-  // other's from 128 tokens on (H 8 / H_kv 2 / D 256, 35229 tokens: 22.3 against 23.1 us); split
-  // over several workgroup columns it shows from the start (H 32 / H_kv 4 / D 128, 8 rows of 512:
-  // 12.5 against 13.3 us).
+  // 172.4). With more heads per lane a wave's arithmetic shows, and from about 100 tokens per split
+  // on two workgroups hide each other's (H 8 / H_kv 2 / D 256, all of them against half: 24576
+  // tokens 19.8 / 18.4 us, 28672 20.5 / 20.7, 30720 19.9 / 21.5); split over several workgroup
+  // columns it shows from the start (H 32 / H_kv 4 / D 128, 8 rows of 512: 12.5 / 13.3).
   p.half = p.n_hchunks == 1 && 4 * B <= p.target / 2 ? p.target / 2 : 0;
-  p.half_max = p.GB <= 2 ? INT32_MAX : 128;
+  p.half_max = p.GB <= 2 ? INT32_MAX : 96;
   p.slots = p.target + B;
   // parked row states of the tsub > 0 rows: (m, l) pairs padded to 16 bytes, then acc
   const size_t parked = size_t(p.TPL - 1) * p.KVB * p.GB;

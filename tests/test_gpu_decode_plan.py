@@ -2,7 +2,7 @@
 token total around the point from which splits have a floor, rows around 32 batches, ragged
 batches whose partial splits overflow the workgroups aimed for (the split size is then fitted),
 64 and 65 rows (fitted or not), and head layouts with one or several workgroup columns and
-with 4 query heads per lane around 128-token splits.
+with 4 query heads per lane around 96-token splits.
 
 Each result is held to the fp32 gather oracle within 2e-2 and, beyond its own 16-bit rounding
 (2^-8 relative for bf16), within 1e-3, the bars of ``test_gpu_decode.py``: a plan that drops,
@@ -59,8 +59,8 @@ CASES = [
     pytest.param(_ragged(33, 1, 900, 8), (32, 16, 128), id="two-columns"),
     pytest.param(_ragged(16, 100, 1500, 9), (32, 4, 128), id="head-chunks"),
     pytest.param(_ragged(30, 1, 1200, 10), (16, 16, 64), id="d64"),
-    pytest.param([2048] * 16, (8, 2, 256), id="4-heads-128-tokens"),
-    pytest.param([2048] * 16 + [9], (8, 2, 256), id="4-heads-past-128-tokens"),
+    pytest.param([2048] * 12, (8, 2, 256), id="4-heads-96-tokens"),
+    pytest.param([2048] * 12 + [9], (8, 2, 256), id="4-heads-past-96-tokens"),
     pytest.param(_ragged(16, 128, 2048, 11), (8, 2, 256), id="4-heads-ragged"),
     pytest.param(_ragged(9, 1, 300, 12), (10, 5, 128), id="five-columns"),
 ]
