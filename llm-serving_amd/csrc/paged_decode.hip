@@ -27,6 +27,7 @@
 //   * software pipeline: block-table entries are loaded two batches ahead and the K/V
 //     registers of the next batch are loaded while the current batch is reduced, so every
 //     wave keeps a batch of loads in flight;
+//   * batches of short rows run one launch with no partials in memory (paged_decode_rows_kernel);
 //   * a row that fits in one split is finished in place; otherwise each split writes its
 //     (m, l, acc) partial to the workspace and a second, small launch folds the partials
 //     with a log-sum-exp merge. (An in-kernel "last split merges" counter needs an
@@ -770,6 +771,230 @@ __global__ __launch_bounds__(256) void paged_decode_merge_kernel(
 }
 #undef MI_PIN8
 
+// One launch instead of two for short rows: one workgroup per (row, KV head, query-head chunk)
+// computes all splits of its row, two or more per wave, and merges them through LDS. Such a
+// launch is latency: this one has the arguments, the row lengths with the row's page ids, and
+// K/V, where the split and merge launches have seven dependent round trips between them; the
+// price is that a row keeps only H_kv CUs busy. Bit-equal to the two launches: the same plan, the
+// same batches, folds and merge order. Measured against them (us per layer, graph replay, H 16 /
+// H_kv 8 / D 128 bf16): 1 row of 16 tokens 6.6 -> 4.6, 4 of 128 7.3 -> 5.9, 8 of 192 9.0 -> 7.2, 32 of
+// 64 9.4 -> 7.2, 32 of 256 12.5 -> 9.8; at the rule's edge 1 of 256 7.0 -> 7.1, 8 of 256 9.1 -> 9.3,
+// beyond it 4 of 320 8.9 -> 9.6. An eager call also saves the second launch's ~4 us on the host.
+template <typename T, int D, int GB, int TPL>
+struct RowsLayout {
+  using Lay = Layout<T, D, GB>;
+  static constexpr int SPW = Lay::RPW >= TPL ? Lay::RPW / TPL : 1;  // splits a wave works on at a time
+  static constexpr int W = 32 / SPW;          // waves: every split of a row at once
+  static constexpr size_t lds(int max_blocks) { return (32 * GB * (D + 2) + size_t(max_blocks)) * sizeof(float); }
+  static constexpr bool ok = sizeof(T) == 2 && GB <= 2 && (D == 64 || D == 128) && Lay::RPW % TPL == 0 && W >= 4 && W <= 16 && GB * D <= 64 * W;
+};
+template <typename T, int D, int GB, int TPL>
+__global__ __launch_bounds__((64 * RowsLayout<T, D, GB, TPL>::W)) void paged_decode_rows_kernel(
+    const T* __restrict__ q, const T* __restrict__ kc, const T* __restrict__ vc,
+    const int32_t* __restrict__ block_table, const int32_t* __restrict__ seqlen, T* __restrict__ out, DecodeArgs a) {
+  using Lay = Layout<T, D, GB>;
+  using Rows = RowsLayout<T, D, GB, TPL>;
+  constexpr int EPL = Lay::EPL, LPR = Lay::LPR, U = Lay::U, SPW = Rows::SPW, W = Rows::W;
+  constexpr int batch = TPL * U, kMost = 32;
+  extern __shared__ float smem[];  // partials [32][GB][D], (m, l) [32][GB][2], page ids
+  float* sm_acc = smem;
+  float* sm_ml = sm_acc + kMost * GB * D;
+  int32_t* sm_pg = reinterpret_cast<int32_t*>(sm_ml + kMost * GB * 2);
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int cols = a.H_kv * a.n_hchunks;
+  const int b = blockIdx.x / cols;
+  const int col = blockIdx.x - b * cols;
+  const int kvh = col / a.n_hchunks, hch = col - kvh * a.n_hchunks;
+  const int h0 = kvh * a.G + hch * GB;
+  const int r = lane / LPR, c = lane - r * LPR;
+  const int tsub = r % TPL;
+  const int capacity = a.max_blocks << a.bs_log2;
+  const int bs_mask = (1 << a.bs_log2) - 1;
+
+  uint4 qr[GB];
+#pragma unroll
+  for (int g = 0; g < GB; ++g) qr[g] = load16(q + b * a.qs0 + (h0 + g) * a.qs1 + c * EPL);
+  // the row's page ids go out with the row lengths (one round trip, not two); entries past the
+  // row's last page are loaded, being inside the table, and never used
+  for (int i = tid; i < a.max_blocks; i += 64 * W) sm_pg[i] = block_table[b * a.bts0 + i];
+  int total = 0, len = 0, len_first = 0;
+  for (int r0 = 0; r0 < a.B; r0 += 64) {
+    const int row = r0 + lane;
+    const int n = row < a.B ? clamp_len(seqlen[row], capacity) : 0;
+    if (r0 == 0) len_first = n;
+    total += __builtin_amdgcn_readlane(wave_inclusive_scan(n), 63);
+    if (b >= r0 && b < r0 + 64) len = __builtin_amdgcn_readlane(n, b - r0);
+  }
+  T* orow = out + b * a.os0 + h0 * a.os1;
+  if (len == 0) {  // uniform
+    for (int i = tid; i < GB * D; i += 64 * W) orow[(i / D) * a.os1 + i % D] = from_f32<T>(0.0f);
+    return;
+  }
+  int n_first, incl;
+  const int chunk = plan_chunk(len_first, total, a, batch, n_first, incl);
+  const int n_split = (len + chunk - 1) / chunk;  // <= 32 (rows_kernel_fits)
+  __syncthreads();
+
+  if (wave * SPW < n_split) {
+    // this lane group's split (past the last one: the last again, not stored)
+    const int sp = wave * SPW + r / TPL;
+    const int s = min(sp, n_split - 1);
+    const int t_begin = s * chunk, t_end = min(len, t_begin + chunk);
+    // the split kernel runs a split's last one or two batches in its masked form, whose rounding
+    // differs (a subtraction where the other has a fused one)
+    const int full = t_begin + ((t_end - t_begin + batch - 1) / batch - 1) / 2 * 2 * batch;
+    const int n_b = (min(chunk, len - wave * SPW * chunk) + batch - 1) / batch;  // of the wave's longest split
+    const T* kbase = kc + kvh * a.ks2 + c * EPL;
+    const T* vbase = vc + kvh * a.vs2 + c * EPL;
+    auto issue = [&](int i, uint4 (&kr)[U], uint4 (&vr)[U]) {
+      int pg[U], off[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int tok = t_begin + i * batch + u * TPL + tsub;
+        const int t = tok < t_end ? tok : t_begin;
+        pg[u] = sm_pg[t >> a.bs_log2];
+        off[u] = t & bs_mask;
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) kr[u] = load_kv(kbase + int64_t(pg[u]) * a.ks0 + off[u] * a.ks1);
+#pragma unroll
+      for (int u = 0; u < U; ++u) vr[u] = load_kv(vbase + int64_t(pg[u]) * a.vs0 + off[u] * a.vs1);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    float m[GB], l[GB], acc[GB][EPL];
+#pragma unroll
+    for (int g = 0; g < GB; ++g) {
+      m[g] = -INFINITY;
+      l[g] = 0.0f;
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) acc[g][e] = 0.0f;
+    }
+    auto compute = [&](int i, const uint4 (&kr)[U], const uint4 (&vr)[U]) {
+      __builtin_amdgcn_sched_barrier(0);
+      const int t0 = t_begin + i * batch;
+      float dot[U][GB], sc[U][GB];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+#pragma unroll
+        for (int g = 0; g < GB; ++g) {
+          dot[u][g] = group_allreduce<LPR, SumOp>(dot16<T>(qr[g], kr[u], 0.0f));
+          sc[u][g] = dot[u][g] * a.scale_log2;
+          if (t0 + u * TPL + tsub >= t_end) sc[u][g] = -INFINITY;
+        }
+      }
+      const bool masked = t0 >= full;
+#pragma unroll
+      for (int g = 0; g < GB; ++g) {
+        float mb = sc[0][g];
+#pragma unroll
+        for (int u = 1; u < U; ++u) mb = fmaxf(mb, sc[u][g]);
+        const float m_new = fmaxf(m[g], mb);
+        const float m_use = m_new == -INFINITY ? 0.0f : m_new;
+        const float alpha = fast_exp2(m[g] - m_use);
+        m[g] = m_new;
+        float lsum_g = l[g] * alpha;
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) acc[g][e] *= alpha;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const float p = fast_exp2(masked ? sc[u][g] - m_use : fmaf(dot[u][g], a.scale_log2, -m_use));
+          lsum_g += p;
+#pragma unroll
+          for (int e = 0; e < EPL; ++e) acc[g][e] = fmaf(p, Vec16<T>::get(vr[u], e), acc[g][e]);
+        }
+        l[g] = lsum_g;
+      }
+    };
+    uint4 kA[U], vA[U], kB[U], vB[U];
+    issue(0, kA, vA);
+    if (n_b > 1) {
+      issue(1, kB, vB);
+      int i = 0;
+      for (; i + 2 < n_b; i += 2) {
+        compute(i, kA, vA);
+        issue(i + 2, kA, vA);
+        compute(i + 1, kB, vB);
+        issue(i + 3, kB, vB);  // past the last batch: clamped to t_begin, dropped
+      }
+      compute(i, kA, vA);
+      if (n_b - i == 2) compute(i + 1, kB, vB);
+    } else {
+      compute(0, kA, vA);
+    }
+    // the TPL states of each split folded in order; the result is the split's partial (or the output
+    // of a row of one split)
+    if constexpr (TPL == 2) {
+      static_assert(LPR == 16 || LPR == 8, "the two states are 16 or 8 lanes apart");
+      auto other = [&](float x, float& x0, float& x1) {  // the tsub 0 and tsub 1 states' values
+        if constexpr (LPR == 16) {
+          const auto w = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+          x0 = __uint_as_float(w[0]);
+          x1 = __uint_as_float(w[1]);
+        } else {
+          const float y = dpp<kDppRowRor8>(x);
+          x0 = tsub == 0 ? x : y;
+          x1 = tsub == 0 ? y : x;
+        }
+      };
+#pragma unroll
+      for (int g = 0; g < GB; ++g) {
+        float m0, m1, l0, l1;
+        other(m[g], m0, m1);
+        other(l[g], l0, l1);
+        const float M = fmaxf(m0, m1);
+        const float Mu = M == -INFINITY ? 0.0f : M;
+        const float w0 = fast_exp2(m0 - Mu), w1 = fast_exp2(m1 - Mu);
+        m[g] = M;
+        l[g] = fmaf(l0, w0, l1 * w1);
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) {
+          float a0, a1;
+          other(acc[g][e], a0, a1);
+          acc[g][e] = fmaf(a0, w0, a1 * w1);
+        }
+      }
+    }
+    if (tsub == 0 && sp < n_split) {
+#pragma unroll
+      for (int g = 0; g < GB; ++g) {
+        if (n_split == 1) {
+          const float inv = 1.0f / fmaxf(l[g], 1.0f);
+          float o[EPL];
+#pragma unroll
+          for (int e = 0; e < EPL; ++e) o[e] = acc[g][e] * inv;
+          store16(orow + g * a.os1 + c * EPL, pack16<T>(o));
+        } else {
+          float4* dst = reinterpret_cast<float4*>(sm_acc + (sp * GB + g) * D + c * EPL);
+#pragma unroll
+          for (int e = 0; e < EPL; e += 4) dst[e / 4] = make_float4(acc[g][e], acc[g][e + 1], acc[g][e + 2], acc[g][e + 3]);
+          if (c == 0) *reinterpret_cast<float2*>(sm_ml + (sp * GB + g) * 2) = make_float2(m[g], l[g]);
+        }
+      }
+    }
+  }
+  if (n_split == 1) return;  // uniform
+  __syncthreads();
+  if (tid >= GB * D) return;  // whole waves; no barrier follows
+  // the merge kernel's arithmetic, thread = (head, element)
+  const int g = tid / D, d = tid - g * D;  // D >= 64: the head is wave-uniform
+  const int j = lane & (kMost - 1);
+  const float2 mlj = *reinterpret_cast<const float2*>(sm_ml + (min(j, n_split - 1) * GB + g) * 2);
+  float v[kMost];
+#pragma unroll
+  for (int k = 0; k < kMost; ++k) v[k] = sm_acc[(min(k, n_split - 1) * GB + g) * D + d];
+  const bool valid = j < n_split;
+  const float M = group_allreduce<kMost, MaxOp>(valid ? mlj.x : -INFINITY);
+  const float Mu = M == -INFINITY ? 0.0f : M;
+  const float w = valid ? fast_exp2(mlj.x - Mu) : 0.0f;
+  const float Ls = group_allreduce<kMost, SumOp>(mlj.y * w);
+  float As = 0.0f;
+#pragma unroll
+  for (int k = 0; k < kMost; ++k) As = fmaf(v[k], __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), k)), As);
+  orow[g * a.os1 + d] = from_f32<T>(As / fmaxf(Ls, 1.0f));
+}
+
 int ilog2_exact(int x) {
   int lg = 0;
   while ((1 << lg) < x) ++lg;
@@ -835,12 +1060,36 @@ Plan make_plan(int B, int H, int H_kv, int D, int block_size, int max_blocks, in
   return p;
 }
 
+// Whether a batch takes the one-launch kernel. Its rows must hold at most 32 splits whatever their
+// lengths: a split is at least a batch long, so 32 batches of table width are the limit (and
+// about where the two launches catch up). Its waves must be resident at once, 16 per CU: 64 rows
+// of 8 KV heads, two rounds of workgroups, took 12.8 against 10.4 us at 64 tokens each.
+bool rows_kernel_fits(const DecodeArgs& a, const Plan& p, int waves) {
+  return (int64_t(a.max_blocks) << a.bs_log2) <= 32 * p.TPL * p.U &&
+         int64_t(a.B) * a.H_kv * a.n_hchunks * waves <= 16 * 256;
+}
+
 template <typename T, int D, int GB>
 int launch_typed(const void* q, const void* kc, const void* vc, const int32_t* bt,
                  const int32_t* seqlen, void* out, int32_t* ws_rows, float* ws_ml,
                  float* ws_acc, const DecodeArgs& a, const Plan& p, const FusedArgs* fa, hipStream_t stream) {
   if (Layout<T, D, GB>::U != p.U || Layout<T, D, GB>::NR != p.NR) {
     return fail(MI_ERR_UNSUPPORTED, "mi_paged_decode: internal launch-geometry mismatch");
+  }
+  auto try_rows = [&](auto tpl) {
+    constexpr int TPL = decltype(tpl)::value;
+    if constexpr (RowsLayout<T, D, GB, TPL>::ok) {
+      using Rows = RowsLayout<T, D, GB, TPL>;
+      if (fa != nullptr || p.TPL != TPL || !rows_kernel_fits(a, p, Rows::W)) return false;
+      hipLaunchKernelGGL((paged_decode_rows_kernel<T, D, GB, TPL>), dim3(a.B * a.H_kv * a.n_hchunks), dim3(64 * Rows::W),
+                         Rows::lds(a.max_blocks), stream, static_cast<const T*>(q), static_cast<const T*>(kc),
+                         static_cast<const T*>(vc), bt, seqlen, static_cast<T*>(out), a);
+      return true;
+    }
+    return false;
+  };
+  if (try_rows(std::integral_constant<int, 2>{}) || try_rows(std::integral_constant<int, 1>{})) {
+    return launch_status("mi_paged_decode (rows kernel)");
   }
   dim3 grid(p.slots, p.n_groups * p.n_hchunks);
   // Wave-uniform pages need every wave inside one token (RPW <= KVB) and the lane byte

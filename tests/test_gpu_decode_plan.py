@@ -1,13 +1,14 @@
 """The decode's device-side split plan at the sizes where it changes its mind: the batch's
 token total around the point from which splits have a floor, rows around 32 batches, ragged
 batches whose partial splits overflow the workgroups aimed for (the split size is then fitted),
-64 and 65 rows (fitted or not), and head layouts with one or several workgroup columns and
-with 4 query heads per lane around 96-token splits.
+64 and 65 rows (fitted or not), head layouts with one or several workgroup columns and with 4
+query heads per lane around 96-token splits, and rows short enough for the one-launch kernel.
 
 Each result is held to the fp32 gather oracle within 2e-2 and, beyond its own 16-bit rounding
 (2^-8 relative for bf16), within 1e-3, the bars of ``test_gpu_decode.py``: a plan that drops,
 repeats or misplaces a split misses them by orders of magnitude. The plan must not depend on
-anything but the row lengths: the same rows through a wider table give the same bits.
+anything but the row lengths, and the one-launch kernel is the two launches' equal bit for bit:
+the same rows through a wider table give the same bits.
 """
 
 from __future__ import annotations
@@ -63,17 +64,31 @@ CASES = [
     pytest.param([2048] * 12 + [9], (8, 2, 256), id="4-heads-past-96-tokens"),
     pytest.param(_ragged(16, 128, 2048, 11), (8, 2, 256), id="4-heads-ragged"),
     pytest.param(_ragged(9, 1, 300, 12), (10, 5, 128), id="five-columns"),
+    # short rows: one launch (table width at most 32 batches)
+    pytest.param([1], QWEN3, id="short-1"),
+    pytest.param([8, 9, 0, 7, 16, 17], QWEN3, id="short-batch-edges"),
+    pytest.param([256, 255, 249, 248, 241, 1], QWEN3, id="short-all-32-splits"),
+    pytest.param(_ragged(32, 0, 256, 13), QWEN3, id="short-32-rows"),
+    pytest.param([250] * 32, QWEN3, id="short-longer-splits"),
+    pytest.param(_ragged(33, 1, 200, 14), QWEN3, id="short-too-many-rows"),
+    pytest.param(_ragged(5, 1, 256, 15), (8, 8, 128), id="short-mha"),
+    pytest.param(_ragged(20, 1, 256, 16), (16, 16, 64), id="short-d64"),
+    pytest.param(_ragged(20, 1, 128, 17), (32, 16, 128), id="short-one-token-loads"),
+    pytest.param(_ragged(3, 1, 128, 18), (32, 32, 64), id="short-d64-one-token-loads"),
+    pytest.param(_ragged(6, 1, 250, 19), (48, 8, 128), id="short-head-chunks"),
 ]
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("lengths,heads", CASES)
-def test_split_plan_edges(lengths, heads, cuda):
+def test_split_plan_edges(lengths, heads, dtype, cuda):
     H, H_kv, D = heads
-    q, k, v, table, seqlen = _build(lengths, H, H_kv, D, torch.bfloat16, seed=len(lengths))
+    q, k, v, table, seqlen = _build(lengths, H, H_kv, D, dtype, seed=len(lengths))
     want = reference_paged_decode(q, k, v, table, seqlen, out_dtype=torch.float32)
     dev = [t.to(cuda) for t in (q, k, v, table, seqlen)]
     got = paged_decode(*dev)
-    wide = torch.cat([dev[3], torch.full((len(lengths), 9), -999, dtype=torch.int32, device=cuda)], 1)
+    # past the short-row kernel's table width: the same rows through the split and merge launches
+    wide = torch.cat([dev[3], torch.full((len(lengths), 17), -999, dtype=torch.int32, device=cuda)], 1)
     again = paged_decode(dev[0], dev[1], dev[2], wide, dev[4])
     torch.cuda.synchronize()
     assert torch.equal(got, again)
