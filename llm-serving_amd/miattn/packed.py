@@ -107,7 +107,8 @@ class PackedPrefill:
         cls._check_sinks(cu, tables)  # one table per prompt
         total, bs = cu[-1], pool.block_size
         host = np.empty(3 * total + len(lengths), dtype=np.int64)
-        host[:total] = np.fromiter(chain.from_iterable(prompts), dtype=np.int64, count=total)
+        # torch.tensor, not numpy: it refuses tokens that are no numbers (numpy would parse strings)
+        host[:total] = torch.tensor(list(chain.from_iterable(prompts)), dtype=torch.long).numpy()
         for t, a, b in zip(tables, cu, cu[1:]):
             at = np.arange(b - a, dtype=np.int64)
             host[total + a: total + b] = at

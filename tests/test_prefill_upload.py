@@ -43,6 +43,7 @@ def test_upload_refuses_what_the_parts_refuse():
     dev = torch.device("cpu")
     for prompts, tables, error in (([[1, 2]], [[9]], IndexError), ([[1] * 17], [[0]], IndexError),
                                    ([[1], [2]], [[0]], ValueError), ([[1], []], [[0], [1]], ValueError),
-                                   ([], [], ValueError), ([[1]], [[True]], ValueError)):
+                                   ([], [], ValueError), ([[1]], [[True]], ValueError),
+                                   ([["1", "2"]], [[0]], ValueError), (["12"], [[0]], ValueError)):
         with pytest.raises(error):
             PackedPrefill.upload(prompts, pool, tables, dev)
