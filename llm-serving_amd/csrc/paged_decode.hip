@@ -706,15 +706,21 @@ __global__ __launch_bounds__(kThreads) void paged_decode_kernel(
 // log-sum-exp merge of their partials, folded online (running max) 32 splits at a time --
 // no LDS, no barrier. Three round trips: the arguments, then the row's length with its
 // (first slot, split count) record written by the first launch, then the partials of up to
-// 32 splits at once (lane j of each 32-lane half loads split j's (m, l), every thread the
-// 32 elements of its d); rows of more than 32 splits take one more per 32. Single-split
+// 16 or of up to 32 splits at once (lane j of each half loads split j's (m, l), every thread
+// the elements of its d); rows of more than 32 splits take one more per 32. Single-split
 // rows were finished by the first launch.
 template <typename T, int D>
 __global__ __launch_bounds__(256) void paged_decode_merge_kernel(
     const int32_t* __restrict__ seqlen, const int32_t* __restrict__ ws_rows,
     const float* __restrict__ ws_ml, const float* __restrict__ ws_acc, T* __restrict__ out,
     DecodeArgs a) {
-  constexpr int kChunk = 32;  // one split per lane of a 32-lane half; the pin names 32
+  constexpr int kChunk = 32;  // one split per lane of a 32-lane half
+  // Rows of up to kFew splits: the wide fold loads and weighs 32 partials whatever their number,
+  // here mostly repeats of the last. Bit-equal (the splits left out weighed 0). Per layer: 32 rows of
+  // 128-2048 tokens 33.2 -> 31.2 us (folds of 8 and 32: 31.8), 16 of 550 12.5 -> 12.2, 100 of 400 35.4 ->
+  // 34.2, 16 of 2048 at H 8 / H_kv 2 / D 256 21.1 -> 20.2; rows of more splits as before (1 of 2048 10.85).
+  // A third fold for up to 8 splits slowed D 256 rows by 1.5%.
+  constexpr int kFew = 16;
   const int h = blockIdx.x;
   const int b = blockIdx.y;
   const int d = threadIdx.x;  // the launch has max(D, 64) threads: whole waves
@@ -742,30 +748,42 @@ __global__ __launch_bounds__(256) void paged_decode_merge_kernel(
   const float* ml = ws_ml + (int64_t(h) * a.slots + first) * 2;  // [head][slot] layout
   const float* acc = ws_acc + (int64_t(h) * a.slots + first) * D + dl;
   float M = -INFINITY, Ls = 0.0f, As = 0.0f;
-  for (int s0 = 0; s0 < n_split; s0 += kChunk) {
-    const int js = s0 + (lane & (kChunk - 1));
+  auto fold = [&](int s0, auto width) {
+    constexpr int N = decltype(width)::value;
+    const int js = s0 + (lane & (N - 1));
     // past the row's last split the loads repeat it (valid memory); weighted out below
     const float2 mlj = *reinterpret_cast<const float2*>(ml + min(js, n_split - 1) * 2);
     float mx = mlj.x, lx = mlj.y;
-    float v[kChunk];
+    float v[N];
 #pragma unroll
-    for (int j = 0; j < kChunk; ++j) v[j] = acc[int64_t(min(s0 + j, n_split - 1)) * D];
+    for (int j = 0; j < N; ++j) v[j] = acc[int64_t(min(s0 + j, n_split - 1)) * D];
     // every load of the chunk is issued before the first wait
-    asm volatile("" : "+v"(mx), "+v"(lx), MI_PIN8("+v", v, 0), MI_PIN8("+v", v, 8),
-                      MI_PIN8("+v", v, 16), MI_PIN8("+v", v, 24));
+    if constexpr (N == 8) {
+      asm volatile("" : "+v"(mx), "+v"(lx), MI_PIN8("+v", v, 0));
+    } else if constexpr (N == 16) {
+      asm volatile("" : "+v"(mx), "+v"(lx), MI_PIN8("+v", v, 0), MI_PIN8("+v", v, 8));
+    } else {
+      asm volatile("" : "+v"(mx), "+v"(lx), MI_PIN8("+v", v, 0), MI_PIN8("+v", v, 8),
+                        MI_PIN8("+v", v, 16), MI_PIN8("+v", v, 24));
+    }
     const bool valid = js < n_split;
-    const float Mc = fmaxf(M, group_allreduce<kChunk, MaxOp>(valid ? mx : -INFINITY));
+    const float Mc = fmaxf(M, group_allreduce<N, MaxOp>(valid ? mx : -INFINITY));
     const float Mu = Mc == -INFINITY ? 0.0f : Mc;
     const float r = fast_exp2(M - Mu);
     const float w = valid ? fast_exp2(mx - Mu) : 0.0f;  // split js's weight, in its lane
-    Ls = fmaf(Ls, r, group_allreduce<kChunk, SumOp>(lx * w));
+    Ls = fmaf(Ls, r, group_allreduce<N, SumOp>(lx * w));
     As *= r;
 #pragma unroll
-    for (int j = 0; j < kChunk; ++j) {
+    for (int j = 0; j < N; ++j) {
       const float wj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), j));
       As = fmaf(v[j], wj, As);
     }
     M = Mc;
+  };
+  if (n_split <= kFew) {
+    fold(0, std::integral_constant<int, kFew>{});
+  } else {
+    for (int s0 = 0; s0 < n_split; s0 += kChunk) fold(s0, std::integral_constant<int, kChunk>{});
   }
   if (d < D) orow[d] = from_f32<T>(As / fmaxf(Ls, 1.0f));
 }

@@ -96,3 +96,26 @@ def test_split_plan_edges(lengths, heads, dtype, cuda):
     assert diff.max().item() <= 2e-2
     assert (diff - want.abs() * 2.0 ** -8).max().item() <= 1e-3
     assert not got[seqlen == 0].any()
+
+
+@pytest.mark.parametrize("lengths", [
+    pytest.param([13, 16, 17], id="2-3-splits"),
+    pytest.param([120, 121, 128, 129], id="15-17-splits"),
+    pytest.param([256, 249], id="32-splits"),
+    pytest.param([257, 511], id="17-32-splits-of-16"),
+    pytest.param([528, 8], id="33-splits"),
+    pytest.param([1, 0, 9, 500], id="mixed"),
+])
+@pytest.mark.parametrize("heads", [QWEN3, (16, 16, 64), (8, 2, 256), (4, 2, 32)], ids=["d128", "d64", "d256", "d32"])
+def test_merge_of_few_and_many_splits(lengths, heads, cuda):
+    """Rows whose split counts lie around the widths that the merge folds at once (16, 32), through
+    a table wide enough that the one-launch kernel does not take them."""
+    H, H_kv, D = heads
+    q, k, v, table, seqlen = _build(lengths, H, H_kv, D, torch.bfloat16, seed=sum(lengths))
+    want = reference_paged_decode(q, k, v, table, seqlen, out_dtype=torch.float32)
+    wide = torch.cat([table, torch.full((len(lengths), 17), -999, dtype=torch.int32)], 1)
+    got = paged_decode(*(t.to(cuda) for t in (q, k, v, wide, seqlen))).cpu()
+    diff = (got.float() - want).abs()
+    assert diff.max().item() <= 2e-2
+    assert (diff - want.abs() * 2.0 ** -8).max().item() <= 1e-3
+    assert not got[seqlen == 0].any()
