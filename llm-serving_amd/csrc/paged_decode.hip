@@ -795,9 +795,10 @@ __global__ __launch_bounds__(256) void paged_decode_merge_kernel(
 // K/V, where the split and merge launches have seven dependent round trips between them; the
 // price is that a row keeps only H_kv CUs busy. Bit-equal to the two launches: the same plan, the
 // same batches, folds and merge order. Measured against them (us per layer, graph replay, H 16 /
-// H_kv 8 / D 128 bf16): 1 row of 16 tokens 6.6 -> 4.6, 4 of 128 7.3 -> 5.9, 8 of 192 9.0 -> 7.2, 32 of
-// 64 9.4 -> 7.2, 32 of 256 12.5 -> 9.8; at the rule's edge 1 of 256 7.0 -> 7.1, 8 of 256 9.1 -> 9.3,
-// beyond it 4 of 320 8.9 -> 9.6. An eager call also saves the second launch's ~4 us on the host.
+// H_kv 8 / D 128 bf16): 1 row of 16 tokens 6.3 -> 4.6, 4 of 128 7.1 -> 5.9, 8 of 192 8.6 -> 7.2, 32 of
+// 64 9.0 -> 7.2, 32 of 256 11.9 -> 9.8; at the rule's edge 1 of 256 7.0 -> 6.8, 16 of 256 9.5 -> 9.7,
+// 8 of 256 8.7 -> 9.3 (kept: an eager call also saves the second launch's ~4 us on the host), beyond it
+// 4 of 320 8.9 -> 9.6.
 template <typename T, int D, int GB, int TPL>
 struct RowsLayout {
   using Lay = Layout<T, D, GB>;
