@@ -192,12 +192,16 @@ constexpr int kSplitFloorLongRow = 16;
 constexpr int kFitSteps = 16;
 
 // Tokens per split of this batch: the splits of all rows (partial ones at the rows' ends counted)
-// fit the workgroups aimed for. A chunk of ceil(total / target) alone overflowed them by up to
-// one split per row, and the CUs that took a workgroup more than the others finished last (32
-// rows of 128-2048 tokens 43.9 -> 36.9 us, 64 rows 62 -> 52 us; batches that happened to fit are
-// as before). Also returns the split count of this lane's row of the first 64 and its inclusive
-// scan. Not fitted: batches past 64 rows (their lengths are not all in registers) and of more
-// than a quarter as many rows as workgroups (their partial splits are no small excess).
+// fit the workgroups aimed for. A chunk of ceil(total / target) alone overflows them by up to
+// one split per row, and the CUs that take a workgroup more than the others finish last (32
+// rows of 128-2048 tokens 43.9 -> 36.9 us, 64 rows 62 -> 52 us, 44 rows of 8192 344 -> 221 us, 64 rows of
+// 4096-8192 369 -> 244 us; batches that happen to fit are unchanged). The chunk grows in steps of a
+// 48th of itself (whole batches), at most kFitSteps = 16 of them, which always suffices: with B rows
+// at most a quarter of the target, 4/3 of total / target is at least total / (target - B), and
+// splits of that size, with one partial split per row, are no more than the target. Also returns
+// the split count of this lane's row of the first 64 and its inclusive scan. Not fitted: batches
+// past 64 rows (their lengths are not all in registers) and of more than a quarter as many rows as
+// workgroups (their partial splits are no small excess).
 __device__ __forceinline__ int plan_chunk(int len_first, int total, const DecodeArgs& a, int batch, int& n, int& incl) {
   // ceil(total / t) in whole batches (a batch is a power of two)
   auto chunk_for = [&](int t, int log2) {
@@ -216,6 +220,7 @@ __device__ __forceinline__ int plan_chunk(int len_first, int total, const Decode
     }
   }
   chunk = max(chunk, batch);
+  const int step = (chunk / (3 * kFitSteps) + batch) & -batch;  // more than a 48th
   for (int i = 0;; ++i) {
     // n = ceil(len / chunk), exact: the quotient is at most a few hundred, so the product is off
     // by less than one either way
@@ -225,7 +230,7 @@ __device__ __forceinline__ int plan_chunk(int len_first, int total, const Decode
     n += r < 0 ? -1 : r >= chunk ? 1 : 0;
     incl = wave_inclusive_scan(n);
     if (i == kFitSteps || a.B > 64 || 4 * a.B > t || __builtin_amdgcn_readlane(incl, 63) <= t) return chunk;
-    chunk += batch;
+    chunk += step;
   }
 }
 

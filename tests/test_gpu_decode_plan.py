@@ -16,7 +16,7 @@ from __future__ import annotations
 import pytest
 import torch
 
-from miattn import paged_decode
+from miattn import _lib, paged_decode
 from oracle.decode import reference_paged_decode
 
 pytestmark = pytest.mark.gpu
@@ -119,3 +119,47 @@ def test_merge_of_few_and_many_splits(lengths, heads, cuda):
     assert diff.max().item() <= 2e-2
     assert (diff - want.abs() * 2.0 ** -8).max().item() <= 1e-3
     assert not got[seqlen == 0].any()
+
+
+def _split_counts(lengths, heads, width=None):
+    """Splits per row, from the (first slot, split count) records that the split launch leaves for the
+    merge at the start of the workspace. Every table entry names one of a few pages, so that long
+    batches cost no memory."""
+    H, H_kv, D = heads
+    B, width = len(lengths), width or -(-max(lengths) // BS)
+    g = torch.Generator().manual_seed(B)
+    k, v = (torch.randn(4, BS, H_kv, D, generator=g).bfloat16().cuda() for _ in range(2))
+    q = torch.randn(B, H, D, generator=g).bfloat16().cuda()
+    table = torch.randint(0, 4, (B, width), generator=g, dtype=torch.int32).cuda()
+    seqlen = torch.tensor(lengths, dtype=torch.int32, device="cuda")
+    out = torch.empty_like(q)
+    code = _lib.dtype_code(q.dtype)
+    n = _lib.lib.mi_paged_decode_workspace_size(B, H, H_kv, D, BS, width, code)
+    ws = torch.full((n,), 0xff, dtype=torch.uint8, device="cuda")
+    rc = _lib.lib.mi_paged_decode(q.data_ptr(), k.data_ptr(), v.data_ptr(), table.data_ptr(), seqlen.data_ptr(),
+                                  out.data_ptr(), B, H, H_kv, D, BS, width,
+                                  _lib.int64_array((*q.stride(), *k.stride(), *v.stride(), *out.stride(), width)),
+                                  D ** -0.5, code, ws.data_ptr(), n, _lib.current_stream(q.device))
+    _lib.check(rc, "mi_paged_decode")
+    torch.cuda.synchronize()
+    some = [0, B // 2, B - 1]
+    want = reference_paged_decode(q[some].cpu(), k.cpu(), v.cpu(), table[some].cpu(), seqlen[some].cpu(),
+                                  out_dtype=torch.float32)
+    assert (out[some].cpu().float() - want).abs().max().item() <= 2e-2
+    return ws[: 8 * B].view(torch.int32).view(B, 2).cpu()
+
+
+@pytest.mark.parametrize("heads,most", [(QWEN3, 256), ((16, 16, 64), 256), ((32, 4, 128), 256), ((8, 2, 256), 512)],
+                         ids=["d128", "d64", "head-chunks", "d256"])
+@pytest.mark.parametrize("lengths", [
+    pytest.param([8192] * 44, id="44x8192"), pytest.param([4096] * 52, id="52x4096"),
+    pytest.param([8192] * 64, id="64x8192"), pytest.param(_ragged(64, 4096, 8192, 20), id="64-ragged"),
+    pytest.param(_ragged(60, 4096, 8192, 21), id="60-ragged"), pytest.param(_ragged(33, 1, 8192, 22), id="33-ragged"),
+    pytest.param([30000] + [5000] * 20, id="one-long"),
+])
+def test_splits_of_long_batches_fit_the_workgroups(lengths, heads, most, cuda):
+    """However long the rows of up to 64 requests are, their splits fit the workgroups aimed for: one
+    workgroup too many puts a second one on a CU that the whole launch then waits for."""
+    first, count = _split_counts(lengths, heads).unbind(1)
+    assert count.sum().item() <= most
+    assert torch.equal(first, count.cumsum(0).int() - count) and count.min().item() >= 1
