@@ -191,6 +191,16 @@ constexpr int kSplitFloor = 24;
 constexpr int kSplitFloorLongRow = 16;
 constexpr int kFitSteps = 16;
 
+// ceil(len / chunk), exact: the quotient is at most a few hundred, so the product is off by less
+// than one either way. (For an integer division the compiler prepares constants of the divisor, on
+// every workgroup's way to its first load, also where only rows past 64 would use them.)
+__device__ __forceinline__ int splits_of(int len, int chunk) {
+  const uint32_t x = uint32_t(len) + uint32_t(chunk) - 1u;
+  const int n = int(float(x) * __builtin_amdgcn_rcpf(float(chunk)));
+  const int r = int(x - uint32_t(n) * uint32_t(chunk));
+  return n + (r < 0 ? -1 : r >= chunk ? 1 : 0);
+}
+
 // Tokens per split of this batch: the splits of all rows (partial ones at the rows' ends counted)
 // fit the workgroups aimed for. A chunk of ceil(total / target) alone overflows them by up to
 // one split per row, and the CUs that take a workgroup more than the others finish last (32
@@ -209,25 +219,19 @@ __device__ __forceinline__ int plan_chunk(int len_first, int total, const Decode
     const uint32_t c = log2 >= 0 ? x >> log2 : x / uint32_t(t);
     return int((c + batch - 1) & -batch);
   };
-  int t = a.target;
-  int chunk = chunk_for(t, a.target_log2);
-  if (a.half > 0) {
-    const int c = chunk_for(a.half, a.half_log2);
-    if (c <= a.half_max) {
-      t = a.half;
-      const int least = total > kTinyTokens ? kSplitFloor : __any(len_first > 32 * batch) ? kSplitFloorLongRow : 0;
-      chunk = max(c, (least + batch - 1) & -batch);
-    }
+  int t = a.half;
+  int chunk = a.half > 0 ? chunk_for(a.half, a.half_log2) : 0;
+  if (a.half > 0 && chunk <= a.half_max) {
+    const int least = total > kTinyTokens ? kSplitFloor : __any(len_first > 32 * batch) ? kSplitFloorLongRow : 0;
+    chunk = max(chunk, (least + batch - 1) & -batch);
+  } else {
+    t = a.target;
+    chunk = chunk_for(a.target, a.target_log2);
   }
   chunk = max(chunk, batch);
   const int step = (chunk / (3 * kFitSteps) + batch) & -batch;  // more than a 48th
   for (int i = 0;; ++i) {
-    // n = ceil(len / chunk), exact: the quotient is at most a few hundred, so the product is off
-    // by less than one either way
-    const uint32_t x = uint32_t(len_first) + uint32_t(chunk) - 1u;
-    n = int(float(x) * __builtin_amdgcn_rcpf(float(chunk)));
-    const int r = int(x - uint32_t(n) * uint32_t(chunk));
-    n += r < 0 ? -1 : r >= chunk ? 1 : 0;
+    n = splits_of(len_first, chunk);
     incl = wave_inclusive_scan(n);
     if (i == kFitSteps || a.B > 64 || 4 * a.B > t || __builtin_amdgcn_readlane(incl, 63) <= t) return chunk;
     chunk += step;
@@ -276,7 +280,7 @@ __device__ __forceinline__ bool plan_split(const int32_t* __restrict__ seqlen, i
     base += __builtin_amdgcn_readlane(incl, 63);
     const int row = r0 + lane;
     len = row < B ? clamp_len(seqlen[row], capacity) : 0;
-    n = (len + chunk - 1) / chunk;
+    n = splits_of(len, chunk);
     incl = wave_inclusive_scan(n);
   }
 }
