@@ -804,10 +804,9 @@ __global__ __launch_bounds__(256) void paged_decode_merge_kernel(
 // K/V, where the split and merge launches have seven dependent round trips between them; the
 // price is that a row keeps only H_kv CUs busy. Bit-equal to the two launches: the same plan, the
 // same batches, folds and merge order. Measured against them (us per layer, graph replay, H 16 /
-// H_kv 8 / D 128 bf16): 1 row of 16 tokens 6.3 -> 4.6, 4 of 128 7.1 -> 5.9, 8 of 192 8.6 -> 7.2, 32 of
-// 64 9.0 -> 7.2, 32 of 256 11.9 -> 9.8; at the rule's edge 1 of 256 7.0 -> 6.8, 16 of 256 9.5 -> 9.7,
-// 8 of 256 8.7 -> 9.3 (kept: an eager call also saves the second launch's ~4 us on the host), beyond it
-// 4 of 320 8.9 -> 9.6.
+// H_kv 8 / D 128 bf16): 1 row of 16 tokens 7.0 -> 5.5, 4 of 128 7.4 -> 6.6, 8 of 192 8.5 -> 7.5, 32 of
+// 64 8.9 -> 6.7, 32 of 192 11.3 -> 9.3 (rows_kernel_fits has the limits of its range); an eager call also
+// saves the second launch's ~4 us on the host.
 template <typename T, int D, int GB, int TPL>
 struct RowsLayout {
   using Lay = Layout<T, D, GB>;
@@ -1088,12 +1087,19 @@ Plan make_plan(int B, int H, int H_kv, int D, int block_size, int max_blocks, in
   return p;
 }
 
-// Whether a batch takes the one-launch kernel. Its rows must hold at most 32 splits whatever their
-// lengths: a split is at least a batch long, so 32 batches of table width are the limit (and
-// about where the two launches catch up). Its waves must be resident at once, 16 per CU: 64 rows
-// of 8 KV heads, two rounds of workgroups, took 12.8 against 10.4 us at 64 tokens each.
-bool rows_kernel_fits(const DecodeArgs& a, const Plan& p, int waves) {
-  return (int64_t(a.max_blocks) << a.bs_log2) <= 32 * p.TPL * p.U &&
+// Whether a batch takes the one-launch kernel. A row's tokens pass through one workgroup per KV head,
+// so the line is the K elements that one may have to stream, 24576 (192 tokens at D 128). Up to there it
+// is the faster one for 1 to 64 rows, even and ragged (H 16 / H_kv 8 / D 128, one launch against two, us
+// per layer in a graph: 1 row of 192 tokens 7.1 / 7.6, 8 of 192 7.5 / 8.5, 32 of up to 192 8.7 / 9.2; at D 64 and
+// with 4-token batches, H 32 / H_kv 16 / D 128, 1.1-1.6x throughout), past it not always (1 of 256 7.8 /
+// 7.6, 32 of up to 256 10.8 / 10.4). 20480 where more than three query-head chunks each stream the row
+// again (H 40 / H_kv 8 / D 128, 2 of 192: 7.6 / 7.45). Its rows must also hold at most 32 splits whatever
+// their lengths, and a split is at least a batch long, so at most 32 batches. Its waves must be resident
+// at once, 16 per CU: 64 rows of 8 KV heads, two rounds of workgroups, took 12.8 against 10.4 us at 64
+// tokens each.
+bool rows_kernel_fits(const DecodeArgs& a, const Plan& p, int D, int waves) {
+  const int64_t capacity = int64_t(a.max_blocks) << a.bs_log2;
+  return capacity * D <= (a.n_hchunks <= 3 ? 24576 : 20480) && capacity <= 32 * p.TPL * p.U &&
          int64_t(a.B) * a.H_kv * a.n_hchunks * waves <= 16 * 256;
 }
 
@@ -1108,7 +1114,7 @@ int launch_typed(const void* q, const void* kc, const void* vc, const int32_t* b
     constexpr int TPL = decltype(tpl)::value;
     if constexpr (RowsLayout<T, D, GB, TPL>::ok) {
       using Rows = RowsLayout<T, D, GB, TPL>;
-      if (fa != nullptr || p.TPL != TPL || !rows_kernel_fits(a, p, Rows::W)) return false;
+      if (fa != nullptr || p.TPL != TPL || !rows_kernel_fits(a, p, D, Rows::W)) return false;
       hipLaunchKernelGGL((paged_decode_rows_kernel<T, D, GB, TPL>), dim3(a.B * a.H_kv * a.n_hchunks), dim3(64 * Rows::W),
                          Rows::lds(a.max_blocks), stream, static_cast<const T*>(q), static_cast<const T*>(kc),
                          static_cast<const T*>(vc), bt, seqlen, static_cast<T*>(out), a);

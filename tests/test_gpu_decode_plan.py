@@ -163,3 +163,20 @@ def test_splits_of_long_batches_fit_the_workgroups(lengths, heads, most, cuda):
     first, count = _split_counts(lengths, heads).unbind(1)
     assert count.sum().item() <= most
     assert torch.equal(first, count.cumsum(0).int() - count) and count.min().item() >= 1
+
+
+@pytest.mark.parametrize("lengths,heads,one_launch", [
+    pytest.param([192], QWEN3, True, id="192"), pytest.param([193], QWEN3, False, id="193"),
+    pytest.param([256, 40, 7, 250, 99, 1, 80, 200], QWEN3, False, id="8-of-256"),
+    pytest.param([192] * 32, QWEN3, True, id="32-of-192"), pytest.param([100] * 33, QWEN3, False, id="too-many-rows"),
+    pytest.param([256], (16, 16, 64), True, id="d64-256"), pytest.param([257], (16, 16, 64), False, id="d64-257"),
+    pytest.param([128], (32, 16, 128), True, id="4-token-batches-128"),
+    pytest.param([129], (32, 16, 128), False, id="4-token-batches-129"),
+    pytest.param([160] * 2, (40, 8, 128), True, id="5-chunks-160"),
+    pytest.param([161] * 2, (40, 8, 128), False, id="5-chunks-161"),
+])
+def test_one_launch_only_where_it_is_the_faster(lengths, heads, one_launch, cuda):
+    """The one-launch kernel leaves no records in the workspace; past its range (tables of more than
+    24576 K elements per row) the two launches run."""
+    records = _split_counts(lengths, heads)
+    assert (records == -1).all().item() if one_launch else (records >= 0).all().item()
