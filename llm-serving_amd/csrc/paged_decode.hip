@@ -47,7 +47,7 @@ namespace miattn {
 namespace {
 
 struct DecodeArgs {
-  int B, H, H_kv, G, kvb_log2, n_hchunks, bs_log2, max_blocks, target, target_log2, half, half_log2, half_max, slots;
+  int B, H, H_kv, G, kvb_log2, n_hchunks, bs_log2, max_blocks, target, target_log2, half, half_log2, half_max, fit, slots;
   int64_t qs0, qs1, ks0, ks1, ks2, vs0, vs1, vs2, os0, os1, bts0;
   float scale_log2;
 };
@@ -208,10 +208,9 @@ __device__ __forceinline__ int splits_of(int len, int chunk) {
 // 4096-8192 369 -> 244 us; batches that happen to fit are unchanged). The chunk grows in steps of a
 // 48th of itself (whole batches), at most kFitSteps = 16 of them, which always suffices: with B rows
 // at most a quarter of the target, 4/3 of total / target is at least total / (target - B), and
-// splits of that size, with one partial split per row, are no more than the target. Also returns
-// the split count of this lane's row of the first 64 and its inclusive scan. Not fitted: batches
-// past 64 rows (their lengths are not all in registers) and of more than a quarter as many rows as
-// workgroups (their partial splits are no small excess).
+// splits of that size, with one partial split per row, are no more than the target. (make_plan says
+// which batches are fitted.) Also returns the split count of this lane's row of the first 64 and its
+// inclusive scan.
 __device__ __forceinline__ int plan_chunk(int len_first, int total, const DecodeArgs& a, int batch, int& n, int& incl) {
   // ceil(total / t) in whole batches (a batch is a power of two)
   auto chunk_for = [&](int t, int log2) {
@@ -219,22 +218,28 @@ __device__ __forceinline__ int plan_chunk(int len_first, int total, const Decode
     const uint32_t c = log2 >= 0 ? x >> log2 : x / uint32_t(t);
     return int((c + batch - 1) & -batch);
   };
-  int t = a.half;
-  int chunk = a.half > 0 ? chunk_for(a.half, a.half_log2) : 0;
-  if (a.half > 0 && chunk <= a.half_max) {
+  bool half = a.half > 0;
+  int chunk = half ? chunk_for(a.half, a.half_log2) : 0;
+  half = half && chunk <= a.half_max;
+  if (half) {
     const int least = total > kTinyTokens ? kSplitFloor : __any(len_first > 32 * batch) ? kSplitFloorLongRow : 0;
     chunk = max(chunk, (least + batch - 1) & -batch);
   } else {
-    t = a.target;
     chunk = chunk_for(a.target, a.target_log2);
   }
   chunk = max(chunk, batch);
-  const int step = (chunk / (3 * kFitSteps) + batch) & -batch;  // more than a 48th
+  int step = (chunk / (3 * kFitSteps) + batch) & -batch;  // more than a 48th
   for (int i = 0;; ++i) {
     n = splits_of(len_first, chunk);
     incl = wave_inclusive_scan(n);
-    if (i == kFitSteps || a.B > 64 || 4 * a.B > t || __builtin_amdgcn_readlane(incl, 63) <= t) return chunk;
+    if (!a.fit || i == kFitSteps || __builtin_amdgcn_readlane(incl, 63) <= (half ? a.half : a.target)) return chunk;
     chunk += step;
+    if (half && chunk > a.half_max) {  // the fitted split is past the range of half the workgroups
+      half = false;
+      chunk = max(chunk_for(a.target, a.target_log2), batch);
+      step = (chunk / (3 * kFitSteps) + batch) & -batch;
+      i = -1;
+    }
   }
 }
 
@@ -1036,7 +1041,7 @@ int lowbit(int x) { return x & -x; }
 
 // Launch geometry, computed identically by the workspace query and the launcher.
 struct Plan {
-  int GB, n_hchunks, KVB, kvb_log2, n_groups, NR, TPL, U, target, half, half_max, slots;
+  int GB, n_hchunks, KVB, kvb_log2, n_groups, NR, TPL, U, target, half, half_max, fit, slots;
   size_t rows_bytes, ml_bytes, acc_bytes;
   size_t smem_bytes;
 };
@@ -1068,14 +1073,22 @@ Plan make_plan(int B, int H, int H_kv, int D, int block_size, int max_blocks, in
   // total / target, and each row adds at most one partial split.
   const int cols = p.n_groups * p.n_hchunks;
   p.target = kTargetSplits / cols > 0 ? kTargetSplits / cols : 1;
+  // The splits are made to fit (plan_chunk) for up to 64 rows (their lengths are in registers) that are at
+  // most a quarter as many as the splits aimed for (their partial splits are a small excess). Not with
+  // more than two workgroup columns: their ranges are short, so a fitted split is a large step above the
+  // exact one, and the columns fill each other's gaps (H 40 / H_kv 8 / D 128, 8 rows of 400: 17.9 us as
+  // they come, 20.1 fitted; H 12 / H_kv 12, 24576 tokens 79.7 / 83.2; with two, H 32 / H_kv 4 and H 32 /
+  // H_kv 32, fitted is 6-14% faster from 8000 tokens on and never slower).
+  p.fit = cols <= 2 && B <= 64 && 4 * B <= p.target;
   // Half of them (one 4-wave workgroup per CU) for splits of up to half_max tokens. With 1 or 2 query
   // heads per lane one workgroup streams as fast as two, and half the splits leave half the
   // merging (16 rows of 256: 11.6 -> 9.9 us per layer, 8 of 2048 19.4 -> 17.1, 32 of 8192 175.5 ->
-  // 172.4). With more heads per lane a wave's arithmetic shows, and from about 100 tokens per split
-  // on two workgroups hide each other's (H 8 / H_kv 2 / D 256, all of them against half: 24576
-  // tokens 19.8 / 18.4 us, 28672 20.5 / 20.7, 30720 19.9 / 21.5); split over several workgroup
-  // columns it shows from the start (H 32 / H_kv 4 / D 128, 8 rows of 512: 12.5 / 13.3).
-  p.half = p.n_hchunks == 1 && 4 * B <= p.target / 2 ? p.target / 2 : 0;
+  // 172.4). With more heads per lane a wave's arithmetic shows, and from about 100 tokens per (fitted)
+  // split on two workgroups hide each other's (H 8 / H_kv 2 / D 256, all of them against half: 24576
+  // tokens 19.8 / 18.4 us, 28672 20.5 / 20.7, 30720 19.9 / 21.5). One column only: the empty workgroups
+  // behind one column's splits scatter the next column's over the CUs, two on some of them (8 rows of
+  // 2048 at H 32 / H_kv 32 / D 128 1.15x slower with half, at H 24 / H_kv 24 / D 64 22.2 / 28.1 us).
+  p.half = cols == 1 && 4 * B <= p.target / 2 ? p.target / 2 : 0;
   p.half_max = p.GB <= 2 ? INT32_MAX : 96;
   p.slots = p.target + B;
   // parked row states of the tsub > 0 rows: (m, l) pairs padded to 16 bytes, then acc
@@ -1273,7 +1286,7 @@ int paged_decode_entry(const void* q, const void* k_cache, const void* v_cache, 
   a.B = B; a.H = H; a.H_kv = H_kv; a.G = H / H_kv; a.kvb_log2 = p.kvb_log2;
   a.n_hchunks = p.n_hchunks; a.bs_log2 = bs_log2;
   a.max_blocks = max_blocks; a.target = p.target; a.target_log2 = ilog2_exact(p.target);
-  a.half = p.half; a.half_log2 = p.half > 0 ? ilog2_exact(p.half) : -1; a.half_max = p.half_max;
+  a.half = p.half; a.half_log2 = p.half > 0 ? ilog2_exact(p.half) : -1; a.half_max = p.half_max; a.fit = p.fit;
   a.slots = p.slots;
   a.qs0 = st[0]; a.qs1 = st[1];
   a.ks0 = st[3]; a.ks1 = st[4]; a.ks2 = st[5];

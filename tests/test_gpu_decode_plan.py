@@ -180,3 +180,22 @@ def test_one_launch_only_where_it_is_the_faster(lengths, heads, one_launch, cuda
     24576 K elements per row) the two launches run."""
     records = _split_counts(lengths, heads)
     assert (records == -1).all().item() if one_launch else (records >= 0).all().item()
+
+
+@pytest.mark.parametrize("heads,lengths,least,most", [
+    # two workgroup columns: all of the workgroups, fitted
+    pytest.param((32, 32, 128), [2048] * 8, 256, 256, id="2-groups"),
+    pytest.param((32, 32, 128), _ragged(20, 1000, 4000, 30), 200, 256, id="2-groups-ragged"),
+    pytest.param((16, 16, 256), [300] * 12, 180, 256, id="2-groups-d256"),
+    # more: as they come, 512 / columns of them and a partial split per row
+    pytest.param((12, 12, 128), [2048] * 8, 140, 178, id="3-groups"),
+    pytest.param((40, 8, 128), [400] * 8, 104, 104, id="5-chunks"),
+    pytest.param((10, 5, 128), [1000] * 10, 80, 80, id="5-groups"),
+    # four heads per lane: half the workgroups up to fitted splits of 96 tokens, all of them past it
+    pytest.param((8, 2, 256), [768] * 32, 256, 256, id="half-96"),
+    pytest.param((8, 2, 256), [2048] * 12, 400, 512, id="half-past-96"),
+])
+def test_workgroups_aimed_for(heads, lengths, least, most, cuda):
+    """How many of the workgroups a batch's splits are shared out over, by the columns of workgroups
+    that its heads need."""
+    assert least <= _split_counts(lengths, heads)[:, 1].sum().item() <= most
