@@ -228,11 +228,15 @@ __device__ __forceinline__ int plan_chunk(int len_first, int total, const Decode
     chunk = chunk_for(a.target, a.target_log2);
   }
   chunk = max(chunk, batch);
-  int step = (chunk / (3 * kFitSteps) + batch) & -batch;  // more than a 48th
-  for (int i = 0;; ++i) {
+  auto count = [&] {
     n = splits_of(len_first, chunk);
     incl = wave_inclusive_scan(n);
-    if (!a.fit || i == kFitSteps || __builtin_amdgcn_readlane(incl, 63) <= (half ? a.half : a.target)) return chunk;
+    return int(__builtin_amdgcn_readlane(incl, 63));
+  };
+  int splits = count();
+  if (!a.fit || splits <= (half ? a.half : a.target)) return chunk;
+  int step = (chunk / (3 * kFitSteps) + batch) & -batch;  // more than a 48th
+  for (int i = 0; i < kFitSteps && splits > (half ? a.half : a.target); ++i) {
     chunk += step;
     if (half && chunk > a.half_max) {  // the fitted split is past the range of half the workgroups
       half = false;
@@ -240,7 +244,9 @@ __device__ __forceinline__ int plan_chunk(int len_first, int total, const Decode
       step = (chunk / (3 * kFitSteps) + batch) & -batch;
       i = -1;
     }
+    splits = count();
   }
+  return chunk;
 }
 
 // This workgroup's piece of the token-balanced split: row b, split index within the row,
