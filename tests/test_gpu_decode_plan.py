@@ -199,3 +199,23 @@ def test_workgroups_aimed_for(heads, lengths, least, most, cuda):
     """How many of the workgroups a batch's splits are shared out over, by the columns of workgroups
     that its heads need."""
     assert least <= _split_counts(lengths, heads)[:, 1].sum().item() <= most
+
+
+@pytest.mark.parametrize("heads,lengths,splits", [
+    # 8-token batches: rows of up to 32 of them are cut by the workgroups alone
+    pytest.param(QWEN3, [256] * 8, [32] * 8, id="32-batches"),
+    pytest.param(QWEN3, [256] * 7 + [257], [11] * 8, id="past-32-batches"),
+    pytest.param(QWEN3, [300], [19], id="tiny"), pytest.param(QWEN3, [1024], [64], id="tiny-edge"),
+    pytest.param(QWEN3, [1025], [43], id="past-tiny"),
+    pytest.param((8, 2, 256), [200] * 6, [25] * 6, id="4-heads"), pytest.param((8, 2, 256), [400] * 3, [17] * 3, id="4-heads-long"),
+    # 4-token batches: floors of two and three of them
+    pytest.param((32, 16, 128), [200], [25], id="4-token-batches"),
+    pytest.param((32, 16, 128), [160] * 7, [14] * 7, id="4-token-batches-past-tiny"),
+    pytest.param((32, 16, 128), [120] * 10, [15] * 10, id="4-token-batches-short"),
+    pytest.param((32, 8, 128), [130, 100], [17, 13], id="4-token-batches-4-heads"),
+    pytest.param((8, 1, 128), [16], [1], id="one-batch"),
+])
+def test_split_floors(heads, lengths, splits, cuda):
+    """Splits per row around the lines of the floors (a table wide enough for the two launches)."""
+    width = max(33, -(-max(lengths) // BS))
+    assert _split_counts(lengths, heads, width)[:, 1].tolist() == splits
