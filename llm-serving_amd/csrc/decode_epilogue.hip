@@ -322,10 +322,24 @@ struct EpilogueArgs {
   float eps; int norm_mode; int32_t* err; hipStream_t s;
 };
 
-// q/k/v values from which the 16-byte kernel runs: below, a launch is latency, and a lane's
-// eight elements are a longer chain than one or two (H 16 / H_kv 8 / D 128: 32 rows 2.75 against
-// 3.28 us, 128 rows 3.17 against 3.45, 256 rows 4.08 against 4.00, 512 rows 6.3 against 5.4).
-constexpr int64_t kVecValues = 1 << 20;
+// Whether the 16-byte kernel is the faster one. Below a number of q/k/v values a launch is latency, and
+// a lane's eight elements are a longer chain than one or two; a row of few heads leaves most of a
+// workgroup empty. bf16 at D 64 and 128: from 2^20 values (H 16 / H_kv 8 / D 128: 256 rows 4.61 -> 4.56 us, 512 6.5 ->
+// 5.6, 8192 64 -> 38) and 8 heads (H 4 / H_kv 2 1.05-1.5x, H 2 / H_kv 1 0.92-1.0x). At D 256 the older kernel's lane has
+// four elements and loses less, least with the Qwen3.5 norm (one division per head, not one per element): H 8 / H_kv
+// 2, 1366 rows 1.06x and 0.98x, 8192 rows 1.18x and 1.07x. fp16 costs a pack for every two roundings and a
+// correction for every quotient (D 128: 2^20 values 0.95-0.99x, 2^21 1.02-1.06x; D 256, H 8 / H_kv 2: 2^24 values 0.99x
+// and 0.93x, 2^26 1.23x).
+template <typename T, int D>
+bool vec_faster(int64_t values, int n_heads, int norm_mode) {
+  const bool bf16 = std::is_same<T, bf16_t>::value, qwen3 = norm_mode == kNormQwen3;
+  if (D == 256) {
+    if (bf16) return n_heads >= 10 && values >= (qwen3 ? int64_t(3) << 20 : int64_t(1) << 24);
+    return n_heads >= 10 && values >= (qwen3 ? int64_t(1) << 25 : int64_t(1) << 26);
+  }
+  if (bf16 || D == 64) return n_heads >= 8 && values >= int64_t(1) << 20;
+  return n_heads >= 10 && values >= int64_t(1) << 21;
+}
 // Rows from which one workgroup walks all heads of a row (8192 rows 39.2 against 45.5 us with
 // the heads shared out over the grid's y axis); below, they are shared out so that a small
 // batch still spreads over the chip (300 rows 4.4 against 5.4 us).
@@ -346,9 +360,10 @@ bool vec16_ok(const EpilogueArgs& a) {
 template <typename T, int D>
 int launch_d(const EpilogueArgs& a) {
   if constexpr (sizeof(T) == 2) {
-    if (a.parts == 0 && int64_t(a.B) * (a.H + 2 * a.H_kv) * D >= kVecValues && vec16_ok(a)) {
+    const int n_heads = a.H + 2 * a.H_kv;
+    if (a.parts == 0 && vec_faster<T, D>(int64_t(a.B) * n_heads * D, n_heads, a.norm_mode) && vec16_ok(a)) {
       constexpr int HPW = 256 * 8 / D;  // heads per workgroup pass
-      const unsigned groups = (a.H + 2 * a.H_kv + HPW - 1) / HPW;
+      const unsigned groups = (n_heads + HPW - 1) / HPW;
       const dim3 grid(a.B, a.B >= kRowPerGroup ? 1 : groups);
       auto go = [&](auto idx_tag) {
         using IdxT = decltype(idx_tag);

@@ -103,3 +103,69 @@ def test_silu_mul_of_many_rows_is_the_small_batches(rows, inter, dtype):
     torch.cuda.synchronize()
     nan = torch.isnan(b)
     assert torch.equal(nan, torch.isnan(a)) and torch.equal(_bits(a)[~nan], _bits(b)[~nan])
+
+
+BF16, FP16 = torch.bfloat16, torch.float16
+
+
+def _epilogue_equals_small_batches(rows, heads, rotary, dtype, zero_centred, pad=None, shift=0):
+    H, H_kv, D = heads
+    g = torch.Generator().manual_seed(rows)
+    width = (H + 2 * H_kv) * D
+    assert rows * width >= 1 << 20
+    if pad is None:
+        pad = 8 if rotary == 64 else 0  # a longer row stride, still 16-byte rows
+    qkv = _values(g, rows, width + pad, dtype=dtype, scale=2.0)[:, shift: shift + width]
+    qn, kn = ((1.0 + 0.1 * torch.randn(D, generator=g)).to(dtype).cuda() for _ in range(2))
+    cos, sin = rope_table(rotary, 1e6, 2048, "cuda", dtype)
+    pos = torch.randint(0, 2048, (rows,), generator=g).cuda()
+    n_blocks = rows // 16 + 2
+    slots = torch.randperm(n_blocks * 16, generator=g)[:rows].to(torch.int32 if pad else torch.int64).cuda()
+    slots[3] = -1                 # nothing to write
+    slots[rows - 2] = n_blocks * 16  # refused: past the pool
+    pos[7] = 2048                 # refused: past the RoPE table
+    got, want = {}, {}
+    for out, step in ((got, rows), (want, 50)):
+        assert step == rows or step * width < 1 << 20
+        pool = PagedPool(1, n_blocks, 16, H_kv, D, dtype=dtype, device="cuda", n_head=H)
+        k, v = (torch.full((rows, H_kv, D), 9.0, dtype=dtype, device="cuda") for _ in range(2))
+        q = []
+        for a in range(0, rows, step):
+            b = min(rows, a + step)
+            q.append(pool.write_qk_norm_rope(0, slots[a:b], qkv[a:b], qn, kn, cos, sin, pos[a:b], 1e-6, k_out=k[a:b],
+                                             v_out=v[a:b], rotary_dim=rotary, zero_centred_norm=zero_centred))
+        torch.cuda.synchronize()
+        out.update(q=torch.cat(q), k=k, v=v, keys=pool.keys[0], values=pool.values[0])
+        with pytest.raises(IndexError):
+            pool.check_writes()
+    for name in got:
+        assert torch.equal(_bits(got[name]), _bits(want[name])), name
+    assert not got["q"][[3, 7, rows - 2]].any() and not got["k"][[3, 7, rows - 2]].any()
+
+
+@pytest.mark.parametrize("rows,heads,rotary,dtype,zero_centred", [
+    # just past the line of each head_dim, type and norm: the 16-byte kernel
+    pytest.param(513, (16, 8, 128), 128, FP16, False, id="d128-fp16"),
+    pytest.param(1040, (16, 8, 128), 64, FP16, True, id="d128-fp16-rows"),
+    pytest.param(343, (16, 16, 64), 64, FP16, True, id="d64-fp16"),
+    pytest.param(2049, (4, 2, 64), 64, BF16, False, id="d64-8-heads"),
+    pytest.param(1025, (8, 2, 256), 64, BF16, False, id="d256"),
+    pytest.param(5462, (8, 2, 256), 64, BF16, True, id="d256-qwen35-norm"),
+    pytest.param(5500, (8, 2, 256), 256, BF16, True, id="d256-qwen35-norm-rot256"),
+    pytest.param(10924, (8, 2, 256), 128, FP16, False, id="d256-fp16"),
+    pytest.param(8193, (16, 8, 256), 64, FP16, True, id="d256-fp16-qwen35-norm"),
+    # just below it, and too few heads: the older kernel in one call and in many
+    pytest.param(511, (16, 8, 128), 128, FP16, False, id="d128-fp16-below"),
+    pytest.param(5461, (8, 2, 256), 64, BF16, True, id="d256-qwen35-norm-below"),
+    pytest.param(2100, (4, 2, 256), 64, BF16, False, id="d256-8-heads"),
+    pytest.param(5500, (1, 1, 64), 64, BF16, False, id="d64-3-heads"),
+])
+def test_epilogue_around_each_line(rows, heads, rotary, dtype, zero_centred):
+    _epilogue_equals_small_batches(rows, heads, rotary, dtype, zero_centred)
+
+
+@pytest.mark.parametrize("pad,shift", [(8, 1), (4, 0), (1, 1), (16, 8)], ids=["pointer", "stride", "both", "aligned"])
+@pytest.mark.parametrize("dtype", [BF16, FP16], ids=["bf16", "fp16"])
+def test_epilogue_of_rows_off_16_bytes(pad, shift, dtype):
+    """A projection whose pointer or row stride is no multiple of 16 bytes goes to the older kernel."""
+    _epilogue_equals_small_batches(530, (16, 8, 128), 128, dtype, False, pad=pad, shift=shift)
