@@ -310,9 +310,17 @@ int launch_norm_per(const void* x, const void* delta, int delta_parts, const voi
   return launch_status("mi_add_rms_norm");
 }
 
-// Rows from which the wave-per-row kernel runs (a quarter of the workgroups: at 128 rows one
-// barrier in 128 workgroups is as fast, 2.8 us, and below that faster).
-constexpr int kWaveRows = 256;
+// Whether the wave-per-row kernel is the faster one (a quarter of the workgroups, no barrier). bf16, with
+// the add: from 256 rows at every width (256 x 1024 3.47 -> 3.12 us, 256 x 4096 7.00 -> 5.44); without it
+// from 320 (256 x 4096 4.33 / 4.46). fp16 costs a pack for every two roundings and a correction for every
+// quotient, so it takes more rows to pay (256 x 4096 4.9 / 6.4, 512 x 3072 0.95x, 1024 rows 1.03x and more at
+// every width), and with the add past 2048 columns, where the older kernel is bound by memory alone, it
+// does not (8192 x 4096 41.4 / 44.3).
+template <typename T>
+bool wave_norm_faster(bool add, int rows, int cols) {
+  if (std::is_same<T, bf16_t>::value) return rows >= (add ? 256 : 320);
+  return rows >= 1024 && (!add || cols <= 2048);
+}
 
 bool aligned16(std::initializer_list<const void*> ps) {
   uintptr_t all = 0;
@@ -324,7 +332,7 @@ template <typename T>
 int launch_norm(const void* x, const void* delta, int delta_parts, const void* w, void* x_out, void* h_out,
                 int rows, int cols, float eps, hipStream_t s) {
   if constexpr (sizeof(T) == 2) {
-    if (rows >= kWaveRows && cols % 512 == 0 && (delta == nullptr || delta_parts == 0) &&
+    if (wave_norm_faster<T>(delta != nullptr, rows, cols) && cols % 512 == 0 && (delta == nullptr || delta_parts == 0) &&
         aligned16({x, delta, w, x_out, h_out})) {
       auto go = [&](auto add, auto ni) {
         hipLaunchKernelGGL((add_rms_norm_wave_kernel<T, decltype(add)::value, decltype(ni)::value>),

@@ -169,3 +169,39 @@ def test_epilogue_around_each_line(rows, heads, rotary, dtype, zero_centred):
 def test_epilogue_of_rows_off_16_bytes(pad, shift, dtype):
     """A projection whose pointer or row stride is no multiple of 16 bytes goes to the older kernel."""
     _epilogue_equals_small_batches(530, (16, 8, 128), 128, dtype, False, pad=pad, shift=shift)
+
+
+def _shifted(t, shift):
+    """``t`` in storage that begins ``shift`` elements past a 16-byte boundary."""
+    flat = torch.empty(t.numel() + shift, dtype=t.dtype, device=t.device)[shift:]
+    return flat.copy_(t.reshape(-1)).view(t.shape)
+
+
+def _add_norm_equals_small_batches(rows, cols, dtype, with_delta, shifts=(0, 0, 0)):
+    g = torch.Generator().manual_seed(rows + cols)
+    x = _values(g, rows, cols, dtype=dtype)
+    d = _shifted(_values(g, rows, cols, dtype=dtype, scale=0.5), shifts[1]) if with_delta else None
+    w = _shifted((1.0 + 0.1 * torch.randn(cols, generator=g)).to(dtype).cuda(), shifts[2])
+    xa, xb = _shifted(x, shifts[0]), x.clone()
+    _, ha = add_rms_norm(xa, d, w, 1e-6)
+    hb = torch.cat([add_rms_norm(xb[a:a + 100], None if d is None else d[a:a + 100], w, 1e-6)[1]
+                    for a in range(0, rows, 100)])
+    torch.cuda.synchronize()
+    assert torch.equal(_bits(xa), _bits(xb)) and torch.equal(_bits(ha), _bits(hb))
+
+
+@pytest.mark.parametrize("rows,cols,dtype,with_delta", [
+    (1024, 512, FP16, True), (1027, 1024, FP16, True), (1025, 1536, FP16, True), (1030, 2048, FP16, True),
+    (1025, 2560, FP16, False), (1024, 3072, FP16, False), (1024, 4096, FP16, False), (1027, 3584, FP16, False),
+    (1030, 2560, FP16, True), (1023, 1024, FP16, True),                        # the older kernel
+    (321, 2048, BF16, False), (257, 2048, BF16, True), (258, 3072, BF16, True), (259, 3584, BF16, True),
+    (300, 1000, BF16, True), (400, 2568, BF16, True), (2000, 1000, FP16, True),  # no multiple of 512
+])
+def test_add_rms_norm_around_each_line(rows, cols, dtype, with_delta):
+    _add_norm_equals_small_batches(rows, cols, dtype, with_delta)
+
+
+@pytest.mark.parametrize("shifts", [(1, 0, 0), (0, 1, 0), (0, 0, 1), (4, 4, 4), (8, 8, 8)])
+@pytest.mark.parametrize("dtype", [BF16, FP16], ids=["bf16", "fp16"])
+def test_add_rms_norm_off_16_bytes(shifts, dtype):
+    _add_norm_equals_small_batches(1030, 1024, dtype, True, shifts)
