@@ -262,8 +262,8 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(ProjIn<T, kU> gu, T* __re
 
 // The same over a T projection with 16-byte accesses (inter % 8 == 0, 16-bit types). Bound by
 // memory (rows x inter x 3 values); the projection is read once, nontemporal. Measured (bf16,
-// inter 3072, graph replay) against the kernel above, one 2-byte element per lane: 8192 rows 59.0
-// -> 29.9 us (151 MB, 5.0 TB/s; a large copy reaches 5.1), 4311 rows 31.8 -> 17.7, 512 rows 4.0 either way.
+// inter 3072, graph replay over the same buffers) against the kernel above, one 2-byte element per lane:
+// 8192 rows 41.3 -> 25.6 us (151 MB), 4096 rows 21.9 -> 14.4, 512 rows 4.3 -> 3.8; fp16 8192 rows 40 -> 28.
 template <typename T>
 __global__ __launch_bounds__(256) void silu_mul_vec_kernel(const T* __restrict__ gu, T* __restrict__ out, int inter) {
   constexpr int E = 8;
@@ -361,15 +361,23 @@ int launch_norm(const void* x, const void* delta, int delta_parts, const void* w
   return launch_norm_per<T, 16>(x, delta, delta_parts, w, x_out, h_out, rows, cols, eps, s);
 }
 
-// Outputs from which the 16-byte silu kernel runs (inter 3072: 32 rows 2.06 against 2.16 us, 128
-// rows 2.24 either way, 256 rows 2.74 against 2.70).
-constexpr int64_t kVecValues = 1 << 19;
+// Outputs from which the 16-byte silu kernel runs, and the narrowest row: below, a launch is latency and
+// the older kernel's eight times as many threads hide it better, or a row leaves most of a workgroup
+// empty.
+template <typename T>
+constexpr int64_t kVecValues = std::is_same<T, bf16_t>::value ? int64_t(1) << 20 : int64_t(1) << 21;
+constexpr int kVecInter = 384;
 
 template <typename T>
 int launch_silu(const void* gu, int gu_parts, void* out, int rows, int inter, hipStream_t s) {
   if constexpr (sizeof(T) == 2) {
-    if (gu_parts == 0 && int64_t(rows) * inter >= kVecValues && inter % 8 == 0 && aligned16({gu, out})) {
-      hipLaunchKernelGGL((silu_mul_vec_kernel<T>), dim3((inter / 8 + 255) / 256, rows), dim3(256), 0, s,
+    if (gu_parts == 0 && int64_t(rows) * inter >= kVecValues<T> && inter >= kVecInter && inter % 8 == 0 &&
+        aligned16({gu, out})) {
+      // a row shared out evenly over workgroups of at most four waves (2560 columns: two of 192 lanes
+      // and not one of 256 with one of 64)
+      const int lanes = inter / 8, groups = (lanes + 255) / 256;
+      const int block = ((lanes + groups - 1) / groups + 63) / 64 * 64;
+      hipLaunchKernelGGL((silu_mul_vec_kernel<T>), dim3((lanes + block - 1) / block, rows), dim3(block), 0, s,
                          static_cast<const T*>(gu), static_cast<T*>(out), inter);
       return launch_status("mi_silu_mul");
     }

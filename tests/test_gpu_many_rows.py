@@ -205,3 +205,19 @@ def test_add_rms_norm_around_each_line(rows, cols, dtype, with_delta):
 @pytest.mark.parametrize("dtype", [BF16, FP16], ids=["bf16", "fp16"])
 def test_add_rms_norm_off_16_bytes(shifts, dtype):
     _add_norm_equals_small_batches(1030, 1024, dtype, True, shifts)
+
+
+@pytest.mark.parametrize("rows,inter,shift", [
+    (2100, 1024, 0), (1001, 3072, 0), (820, 2560, 0), (5500, 384, 0), (260, 8200, 0), (2731, 776, 0), (1366, 1544, 0),
+    (5700, 376, 0), (2100, 1004, 0),                       # narrow, or no multiple of 8
+    (2100, 1024, 1), (2100, 1024, 4), (2100, 1024, 8),     # off 16 bytes, and on them again
+])
+@pytest.mark.parametrize("dtype", [BF16, FP16], ids=["bf16", "fp16"])
+def test_silu_mul_around_each_line(rows, inter, shift, dtype):
+    g = torch.Generator().manual_seed(rows)
+    assert rows * inter >= 1 << 21
+    gu = _shifted(_values(g, rows, 2 * inter, dtype=dtype, scale=3.0), shift)
+    step = max(1, (1 << 18) // inter)
+    a, b = silu_mul(gu), torch.cat([silu_mul(gu[i:i + step].clone()) for i in range(0, rows, step)])
+    torch.cuda.synchronize()
+    assert torch.equal(_bits(a), _bits(b))
