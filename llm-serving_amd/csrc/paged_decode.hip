@@ -574,9 +574,11 @@ __global__ __launch_bounds__(kThreads) void paged_decode_kernel(
 
   // Online softmax over one batch of U tokens per row state. Only a split's last batch
   // can hold tokens past t_end, so the steady-state loop runs the unmasked form.
+  // Its exponents are one fused operation each; the masked form subtracts from the rounded score
+  // (paged_decode_rows_kernel, which must give the same bits, does both likewise).
   auto compute = [&](int t0, const uint4 (&kr)[U], const uint4 (&vr)[U], auto masked) {
     __builtin_amdgcn_sched_barrier(0);
-    float s[U][GB];
+    float dots[U][GB], s[U][GB];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
 #pragma unroll
@@ -587,6 +589,7 @@ __global__ __launch_bounds__(kThreads) void paged_decode_kernel(
         }
         float dot = dot16<T>(qr[g], kk, 0.0f);
         dot = group_allreduce<LPR, SumOp>(dot);
+        dots[u][g] = dot;
         s[u][g] = dot * a.scale_log2;
         if constexpr (decltype(masked)::value) {
           if (t0 + u * TPL + tsub >= t_end) s[u][g] = -INFINITY;
@@ -607,7 +610,9 @@ __global__ __launch_bounds__(kThreads) void paged_decode_kernel(
       for (int e = 0; e < EPL; ++e) acc[g][e] *= alpha;
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        const float p = fast_exp2(s[u][g] - m_use);
+        float x = s[u][g] - m_use;
+        if constexpr (!decltype(masked)::value) x = fmaf(dots[u][g], a.scale_log2, -m_use);
+        const float p = fast_exp2(x);
         lsum_g += p;
         uint4 vv = vr[u];
         if constexpr (kFused && decltype(masked)::value) {
@@ -887,8 +892,8 @@ __global__ __launch_bounds__((64 * RowsLayout<T, D, GB, TPL>::W)) void paged_dec
     const int sp = wave * SPW + r / TPL;
     const int s = min(sp, n_split - 1);
     const int t_begin = s * chunk, t_end = min(len, t_begin + chunk);
-    // the split kernel runs a split's last one or two batches in its masked form, whose rounding
-    // differs (a subtraction where the other has a fused one)
+    // the split kernel runs a split's last one or two batches in its masked form, whose exponents
+    // round the score first
     const int full = t_begin + ((t_end - t_begin + batch - 1) / batch - 1) / 2 * 2 * batch;
     const int n_b = (min(chunk, len - wave * SPW * chunk) + batch - 1) / batch;  // of the wave's longest split
     const T* kbase = kc + kvh * a.ks2 + c * EPL;
