@@ -280,7 +280,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_write_vec_kernel(
         for (int j = 0; j < E; ++j) x[j] = (x[j] * r) * (1.0f + Vec16<T>::get(w, j));
       }
       result = rt8<T>(x);  // the normed head
-      if (e0 < rotary || half == 128) {
+      if (e0 < rotary) {
         // the rotation partner is this element of lane c ^ (half / 8); the first half's lanes take
         // x cos - partner sin, the second's partner sin + x cos
         float p[E];

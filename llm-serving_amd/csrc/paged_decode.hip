@@ -790,9 +790,7 @@ __global__ __launch_bounds__(256) void paged_decode_merge_kernel(
 #pragma unroll
     for (int j = 0; j < N; ++j) v[j] = acc[int64_t(min(s0 + j, n_split - 1)) * D];
     // every load of the chunk is issued before the first wait
-    if constexpr (N == 8) {
-      asm volatile("" : "+v"(mx), "+v"(lx), MI_PIN8("+v", v, 0));
-    } else if constexpr (N == 16) {
+    if constexpr (N == 16) {
       asm volatile("" : "+v"(mx), "+v"(lx), MI_PIN8("+v", v, 0), MI_PIN8("+v", v, 8));
     } else {
       asm volatile("" : "+v"(mx), "+v"(lx), MI_PIN8("+v", v, 0), MI_PIN8("+v", v, 8),
