@@ -144,3 +144,13 @@ def test_fused_other_head_groupings(heads):
     launches."""
     pools, out_a, out_b = _both(_case([5, 700, 33, 1500, 129], parts=2, seed=13, heads=heads))
     _assert_same(pools, out_a, out_b)
+
+
+@pytest.mark.parametrize("parts", [0, 2], ids=["plain", "parts2"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_fused_of_a_short_table_equals_the_one_launch_decode(parts, dtype):
+    """A table of at most 192 tokens: ``run`` takes the one-launch kernel there, the fused form its
+    split and merge launches."""
+    pools, out_a, out_b = _both(_case([1, 2, 15, 16, 17, 33, 190, 1, 64, 129], parts=parts, dtype=dtype, seed=17, idle=(3,)))
+    _assert_same(pools, out_a, out_b)
+    assert not out_b[3].any()

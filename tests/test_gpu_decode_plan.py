@@ -16,7 +16,7 @@ from __future__ import annotations
 import pytest
 import torch
 
-from miattn import _lib, paged_decode
+from miattn import _lib, paged_decode, paged_decode_plan
 from oracle.decode import reference_paged_decode
 
 pytestmark = pytest.mark.gpu
@@ -219,3 +219,81 @@ def test_split_floors(heads, lengths, splits, cuda):
     """Splits per row around the lines of the floors (a table wide enough for the two launches)."""
     width = max(33, -(-max(lengths) // BS))
     assert _split_counts(lengths, heads, width)[:, 1].tolist() == splits
+
+
+def _other_pools(k, v, table, seqlen, block, head_major):
+    """The same rows over pools of another page size, each page's tokens moved, and of another layout."""
+    lengths, H_kv, D = seqlen.tolist(), k.shape[2], k.shape[3]
+    need = [max(1, -(-n // block)) for n in lengths]
+    n_blocks = sum(need) + 2
+    k2, v2 = (torch.full((n_blocks, block, H_kv, D), 7.0, dtype=k.dtype) for _ in range(2))
+    table2 = torch.zeros(len(lengths), max(need), dtype=torch.int32)
+    ids = torch.randperm(n_blocks, generator=torch.Generator().manual_seed(block)).tolist()
+    for r, n in enumerate(lengths):
+        for page in range(need[r]):
+            table2[r, page] = ids.pop()
+        for old, new in ((k, k2), (v, v2)):
+            row = old[table[r].long()].reshape(-1, H_kv, D)[:n]
+            for page in range(-(-n // block)):
+                part = row[page * block:(page + 1) * block]
+                new[int(table2[r, page]), : len(part)] = part
+    if head_major:
+        k2, v2 = (t.permute(0, 2, 1, 3).contiguous().permute(0, 2, 1, 3) for t in (k2, v2))
+    return k2.cuda(), v2.cuda(), table2.cuda()
+
+
+@pytest.mark.parametrize("head_major", [False, True], ids=["token-major", "head-major"])
+@pytest.mark.parametrize("block", [1, 4, 16, 32, 64])
+@pytest.mark.parametrize("heads,lengths", [
+    pytest.param(QWEN3, [1, 0, 150, 64, 33, 97, 128], id="d128"),
+    pytest.param((16, 16, 64), [1, 150, 190, 64, 0, 65], id="d64"),
+    pytest.param((32, 16, 128), [1, 100, 64, 0, 128], id="4-token-batches"),
+    pytest.param((48, 8, 128), [128, 5, 77], id="head-chunks"),
+])
+def test_one_launch_of_other_pages_and_layouts(heads, lengths, block, head_major, cuda):
+    H, H_kv, D = heads
+    q, k, v, table, seqlen = _build(lengths, H, H_kv, D, torch.bfloat16, seed=sum(lengths))
+    ref = paged_decode(*(t.cuda() for t in (q, k, v)), torch.cat(
+        [table, torch.full((len(lengths), 17), -999, dtype=torch.int32)], 1).cuda(), seqlen.cuda())  # two launches
+    k2, v2, table2 = _other_pools(k, v, table, seqlen, block, head_major)
+    assert block * table2.shape[1] * D <= 24576
+    got = paged_decode(q.cuda(), k2, v2, table2, seqlen.cuda())
+    torch.cuda.synchronize()
+    assert torch.equal(got, ref)
+    want = reference_paged_decode(q, k, v, table, seqlen, out_dtype=torch.float32)
+    assert (got.cpu().float() - want).abs().max().item() <= 2e-2
+
+
+def test_one_launch_in_a_graph_whose_rows_grow(cuda):
+    """A captured call reads the row lengths at each replay: rows grow, start and end between replays."""
+    H, H_kv, D = QWEN3
+    q, k, v, table, _ = _build([192] * 6, H, H_kv, D, torch.bfloat16, seed=5)
+    q, k, v, table = (t.cuda() for t in (q, k, v, table))
+    wide = torch.cat([table, torch.full((6, 17), -999, dtype=torch.int32, device=cuda)], 1)
+    seqlen = torch.tensor([1, 8, 0, 100, 16, 191], dtype=torch.int32, device=cuda)
+    plan = paged_decode_plan(q, [k], [v], table, seqlen)
+    plan.run(0, q)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = plan.run(0, q)
+    for step, lengths in enumerate([[1, 8, 0, 100, 16, 191], [2, 9, 1, 101, 17, 192], [8, 16, 64, 128, 24, 0],
+                                    [0, 0, 0, 0, 0, 0], [192] * 6, [192, 1, 1, 1, 1, 1]]):
+        seqlen.copy_(torch.tensor(lengths, dtype=torch.int32))
+        out.fill_(9.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, paged_decode(q, k, v, wide, seqlen)), step
+        assert not out[seqlen == 0].any()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("lengths,heads", [
+    pytest.param([192, 191, 185, 184, 177, 1], QWEN3, id="24-splits"),
+    pytest.param([190] * 32, QWEN3, id="32-rows-longer-splits"), pytest.param(_ragged(32, 0, 192, 40), QWEN3, id="32-ragged"),
+    pytest.param([256, 255, 249, 1], (16, 16, 64), id="d64-32-splits"),
+    pytest.param([128, 127, 125, 124, 1], (32, 16, 128), id="4-token-batches-32-splits"),
+    pytest.param([160, 33], (40, 8, 128), id="5-chunks"), pytest.param(_ragged(7, 1, 192, 41), (8, 8, 128), id="one-head"),
+])
+def test_one_launch_up_to_its_widest_table(lengths, heads, dtype, cuda):
+    test_split_plan_edges(lengths, heads, dtype, cuda)
