@@ -108,7 +108,10 @@ class PackedPrefill:
         total, bs = cu[-1], pool.block_size
         host = np.empty(3 * total + len(lengths), dtype=np.int64)
         # torch.tensor, not numpy: it refuses tokens that are no numbers (numpy would parse strings)
-        host[:total] = torch.tensor(list(chain.from_iterable(prompts)), dtype=torch.long).numpy()
+        flat = torch.tensor(list(chain.from_iterable(prompts)), dtype=torch.long)
+        if flat.shape != (total,):  # numpy would drop the dimensions of a lone nested token
+            raise ValueError(f"prompts must be sequences of tokens, got {tuple(flat.shape)} for {total} tokens")
+        host[:total] = flat.numpy()
         for t, a, b in zip(tables, cu, cu[1:]):
             at = np.arange(b - a, dtype=np.int64)
             host[total + a: total + b] = at

@@ -47,3 +47,10 @@ def test_upload_refuses_what_the_parts_refuse():
                                    ([["1", "2"]], [[0]], ValueError), (["12"], [[0]], ValueError)):
         with pytest.raises(error):
             PackedPrefill.upload(prompts, pool, tables, dev)
+
+
+@pytest.mark.parametrize("prompts", [[[[5]]], [[[5], [6]]], [[[5, 6]]]])
+def test_upload_refuses_nested_tokens(prompts):
+    """Refused by the packed tensor's shape before, one token or several."""
+    with pytest.raises(ValueError):
+        PackedPrefill.upload(prompts, PagedPool(1, 4, 16, 2, 8), [[0]], torch.device("cpu"))
