@@ -89,8 +89,9 @@ class PackedPrefill:
     def upload(cls, prompts: Sequence[Sequence[int]], pool, block_tables, device):
         """The container of whole prompts written into one paged ``pool``, and their packed tokens.
         What the group needs on the device -- tokens, request-local positions, slot map, last
-        indices -- is built on the host and uploaded in one copy; nothing is read back, so the
-        host does not wait for work already queued."""
+        indices -- is built on the host and uploaded in one copy. It is a blocking copy from
+        pageable memory, so the host waits once for the work already queued on the stream;
+        nothing is read back."""
         from .paged import PagedWriteSink
 
         lengths = [len(p) for p in prompts]
