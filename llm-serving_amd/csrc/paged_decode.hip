@@ -1096,16 +1096,25 @@ Plan make_plan(int B, int H, int H_kv, int D, int block_size, int max_blocks, in
   // they come, 20.1 fitted; H 12 / H_kv 12, 24576 tokens 79.7 / 83.2; with two, H 32 / H_kv 4 and H 32 /
   // H_kv 32, fitted is 6-14% faster from 8000 tokens on and never slower).
   p.fit = cols <= 2 && B <= 64 && 4 * B <= p.target;
-  // Half of them (one 4-wave workgroup per CU) for splits of up to half_max tokens. With 1 or 2 query
-  // heads per lane one workgroup streams as fast as two, and half the splits leave half the
-  // merging (16 rows of 256: 11.6 -> 9.9 us per layer, 8 of 2048 19.4 -> 17.1, 32 of 8192 175.5 ->
-  // 172.4). With more heads per lane a wave's arithmetic shows, and from about 100 tokens per (fitted)
-  // split on two workgroups hide each other's (H 8 / H_kv 2 / D 256, all of them against half: 24576
-  // tokens 19.8 / 18.4 us, 28672 20.5 / 20.7, 30720 19.9 / 21.5). One column only: the empty workgroups
-  // behind one column's splits scatter the next column's over the CUs, two on some of them (8 rows of
-  // 2048 at H 32 / H_kv 32 / D 128 1.15x slower with half, at H 24 / H_kv 24 / D 64 22.2 / 28.1 us).
+  // Half of them (one 4-wave workgroup per CU) for (fitted) splits of up to half_max tokens: half the
+  // splits leave half the merging (16 rows of 256: 11.6 -> 9.9 us per layer, 8 of 2048 19.4 -> 17.1, 32 of
+  // 8192 175.5 -> 172.4), and with 1 or 2 query heads per lane and wave-uniform pages one workgroup
+  // streams as fast as two. Where a batch of loads is more of a latency, two hide each other's, and the
+  // more batches a split has the more that is worth: with 4 heads per lane past 24 batches (12 where a
+  // row of D takes more than 16 lanes), with 8 past 8 (4 where it takes a whole wave), with a page id per
+  // lane, loaded in line with K and V, past 8 and, with 1 or 2 heads, past 3. Measured, half against
+  // the plan before it, even rows, at 4 / 16 / 64 batches: H 16 / H_kv 8 / D 128 0.86 / 0.94 / 0.96, H 32 /
+  // H_kv 8 0.78 / 0.89 / 0.98, H 8 / H_kv 2 / D 256 0.83 / 0.97 / 1.09, H 4 / H_kv 1 / D 128 (page ids per lane) 0.81 /
+  // 0.96 / 1.17, H 2 / H_kv 2 / D 128 (likewise) 0.99 / 1.03 / 1.03, fp32 H 64 / H_kv 8 / D 128 (8 heads) 0.81 / 1.02 /
+  // 1.25; all of them 0.98-1.01 throughout. One column only: the empty workgroups behind one column's splits
+  // scatter the next column's over the CUs, two on some of them (8 rows of 2048 at H 32 / H_kv 32 / D 128 1.15x
+  // slower with half, at H 24 / H_kv 24 / D 64 22.2 / 28.1 us).
   p.half = cols == 1 && 4 * B <= p.target / 2 ? p.target / 2 : 0;
-  p.half_max = p.GB <= 2 ? INT32_MAX : 96;
+  const bool uniform_pages = 64 / lpr <= p.KVB;
+  const int half_batches = p.GB <= 2 ? (uniform_pages ? INT32_MAX : 3)
+                           : p.GB == 4 ? (!uniform_pages ? 8 : lpr <= 16 ? 24 : 12)
+                                       : (lpr <= 32 ? 8 : 4);
+  p.half_max = half_batches == INT32_MAX ? INT32_MAX : half_batches * p.TPL * p.U;
   p.slots = p.target + B;
   // parked row states of the tsub > 0 rows: (m, l) pairs padded to 16 bytes, then acc
   const size_t parked = size_t(p.TPL - 1) * p.KVB * p.GB;

@@ -191,9 +191,16 @@ def test_one_launch_only_where_it_is_the_faster(lengths, heads, one_launch, cuda
     pytest.param((12, 12, 128), [2048] * 8, 140, 178, id="3-groups"),
     pytest.param((40, 8, 128), [400] * 8, 104, 104, id="5-chunks"),
     pytest.param((10, 5, 128), [1000] * 10, 80, 80, id="5-groups"),
-    # four heads per lane: half the workgroups up to fitted splits of 96 tokens, all of them past it
-    pytest.param((8, 2, 256), [768] * 32, 256, 256, id="half-96"),
-    pytest.param((8, 2, 256), [2048] * 12, 400, 512, id="half-past-96"),
+    # half the workgroups up to fitted splits of so many batches, all of them past it: four heads per
+    # lane at D 256 (12 of 8 tokens) and at D 128 (24 of 4 tokens), page ids per lane (8 of 32; 3 of 32)
+    pytest.param((8, 2, 256), [1536] * 16, 256, 256, id="d256-12-batches"),
+    pytest.param((8, 2, 256), [2048] * 12, 400, 512, id="d256-fitted-past-12"),
+    pytest.param((32, 8, 128), [768] * 32, 256, 256, id="gqa4-24-batches"),
+    pytest.param((32, 8, 128), [800] * 32, 400, 512, id="gqa4-past-24"),
+    pytest.param((4, 1, 128), [2048] * 32, 256, 256, id="one-kv-head-8-batches"),
+    pytest.param((4, 1, 128), [2100] * 32, 400, 512, id="one-kv-head-past-8"),
+    pytest.param((2, 2, 128), [1536] * 16, 256, 256, id="two-kv-heads-3-batches"),
+    pytest.param((2, 2, 128), [1600] * 16, 400, 512, id="two-kv-heads-past-3"),
 ])
 def test_workgroups_aimed_for(heads, lengths, least, most, cuda):
     """How many of the workgroups a batch's splits are shared out over, by the columns of workgroups
