@@ -307,9 +307,12 @@ __device__ __forceinline__ bool plan_split(const int32_t* __restrict__ seqlen, i
 // (rows per wave <= KV heads per group, true at the Qwen3 shape), so the block-table
 // entries are wave-uniform and read with scalar loads. Those are counted apart from the
 // K/V vector loads, so the in-order vector-load counter tracks only K/V batches and the
-// reduction of batch i never waits for batch i+1.
+// reduction of batch i never waits for batch i+1. Up to 4 heads per lane that form fits in the registers
+// of four workgroups per CU, which a batch with more splits than two per CU runs at once; left to
+// itself the compiler takes one too many with 4 bf16 heads (129; H 128 / H_kv 8 / D 256, 99 rows of 1032: 643 us
+// per layer at four, 754 at three).
 template <typename T, int D, int GB, bool UP, bool kFused>
-__global__ __launch_bounds__(kThreads) void paged_decode_kernel(
+__global__ __launch_bounds__(kThreads, UP && !kFused && GB <= 4 ? 4 : 1) void paged_decode_kernel(
     const T* __restrict__ q, const T* __restrict__ kc, const T* __restrict__ vc,
     const int32_t* __restrict__ block_table, const int32_t* __restrict__ seqlen,
     T* __restrict__ out, int32_t* __restrict__ ws_rows, float* __restrict__ ws_ml,
